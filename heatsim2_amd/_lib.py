@@ -14,6 +14,7 @@ LIB_PATH = os.path.join(HERE, "libhs2.so")
 
 HS2_OK = 0
 HS2_OPT_COMBINED_X = 1
+HS2_OPT_LINE_TABLES = 2
 # the version string hs2_version() of a matching libhs2.so starts with
 LIBRARY_VERSION = "0.5"
 _ERRNAMES = {1: "HS2_E_ARG", 2: "HS2_E_UNSUPPORTED", 3: "HS2_E_HIP", 4: "HS2_E_STATE",
@@ -35,7 +36,7 @@ class HS2Error(RuntimeError):
 # every symbol include/heatsim2_amd.h declares
 EXPORTS = ("hs2_plan_create", "hs2_plan_destroy", "hs2_plan_set_compact", "hs2_plan_set_dense",
            "hs2_plan_set_dense_asym", "hs2_plan_expand", "hs2_plan_set_config", "hs2_plan_set_option",
-           "hs2_plan_info",
+           "hs2_plan_get_option", "hs2_plan_info",
            "hs2_step", "hs2_run",
            "hs2_run_timed", "hs2_grad_work_doubles", "hs2_grad_forward", "hs2_grad_backward",
            "hs2_batch_create", "hs2_batch_destroy", "hs2_batch_layout", "hs2_batch_set_dense",
@@ -71,6 +72,8 @@ def load():
     L.hs2_plan_set_config.restype = i32
     L.hs2_plan_set_option.argtypes = [vp, i32, i32]
     L.hs2_plan_set_option.restype = i32
+    L.hs2_plan_get_option.argtypes = [vp, i32, ctypes.POINTER(i32)]
+    L.hs2_plan_get_option.restype = i32
     L.hs2_plan_info.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
     L.hs2_plan_info.restype = i32
     L.hs2_step.argtypes = [vp, vp, vp, vp, vp, i32, vp, vp, vp]

@@ -6,7 +6,9 @@ segment, lines per block) -- i.e. how much of each line is eliminated
 Thomas-style in registers and how much goes to the parallel cyclic
 reduction across lanes / threads.  Candidates are timed on
 the device with HIP events (hs2_run_timed) on a scratch copy of the field;
-the fastest of each sweep is set on the plan.  Results are cached per
+the fastest of each sweep is set on the plan.  These shapes are the class-map
+and per-cell kernels'; a plan with line tables (HS2_OPT_LINE_TABLES) is timed
+with them as well and keeps whichever is faster.  Results are cached per
 (device name, grid shape, coefficient mode) in memory and, if writable, in
 $HS2_TUNE_CACHE (default ~/.cache/heatsim2_amd/tune.json).
 
@@ -99,13 +101,15 @@ def _time(L, plan, T, steps):
 def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
     """Pick and set the fastest launch shapes for this plan; returns
     {"x": (cpl, lanes, lines, tile rows), "y": (seg, lines), "z": (seg, lines),
-    "ms": [x, y, z]}."""
+    "ms": [x, y, z], "lines": whether the plan's line tables are used instead}."""
     L = _lib.load()
     plan = ADI_params.plan
     nz, ny, nx = ADI_params.shape
     info = _lib.plan_info(plan)
-    key = "%s|%s|%dx%dx%d|mode%d" % (L.hs2_version().decode(), torch.cuda.get_device_name(),
-                                     nz, ny, nx, info["mode"])
+    lines = _line_tables(L, plan)
+    key = "%s|%s|%dx%dx%d|mode%d|lines%d" % (L.hs2_version().decode(),
+                                             torch.cuda.get_device_name(), nz, ny, nx,
+                                             info["mode"], lines)
     if use_cache:
         cfg = _memo.get(key) or _load_cache().get(key)
         if cfg and _apply(L, plan, cfg, strict=False):
@@ -142,7 +146,22 @@ def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
             cur[axis_name] = cand
         _apply(L, plan, cur)
         best_ms[idx] = _time(L, plan, scratch, steps)[idx] if results else None
-    cfg = {"x": list(cur["x"]), "y": list(cur["y"]), "z": list(cur["z"]), "ms": best_ms}
+    cfg = {"x": list(cur["x"]), "y": list(cur["y"]), "z": list(cur["z"]), "ms": best_ms,
+           "lines": False}
+    if lines:
+        # each side the fastest of three, in turn
+        t = {True: [], False: []}
+        for _ in range(3):
+            for on in (True, False):
+                _set_lines(L, plan, on)
+                t[on].append(_time(L, plan, scratch, steps))
+        best = {on: min(v, key=sum) for on, v in t.items()}
+        if verbose:
+            print("autotune line tables: %s ms against %s" % (best[True], best[False]), flush=True)
+        cfg["lines"] = sum(best[True]) < sum(best[False])
+        if cfg["lines"]:
+            cfg["ms"] = best[True]
+        _set_lines(L, plan, cfg["lines"])
     _memo[key] = cfg
     if use_cache:
         _store_cache(key, cfg)
@@ -157,4 +176,26 @@ def _apply(L, plan, cfg, strict=True):
                                int(cfg["z"][1]))
     if strict:
         _lib.check("hs2_plan_set_config", rc)
+    if rc == 0 and cfg.get("lines"):
+        _set_lines(L, plan, True)
     return rc == 0
+
+
+def _set_lines(L, plan, on):
+    _lib.check("hs2_plan_set_option",
+               L.hs2_plan_set_option(plan, _lib.HS2_OPT_LINE_TABLES, int(on)))
+
+
+def _line_tables(L, plan):
+    """The axes the plan has line tables for, whether or not it uses them."""
+    axes = ctypes.c_int()
+
+    def get():
+        _lib.check("hs2_plan_get_option",
+                   L.hs2_plan_get_option(plan, _lib.HS2_OPT_LINE_TABLES, ctypes.byref(axes)))
+        return axes.value
+    if not get():
+        _set_lines(L, plan, True)
+        get()
+        _set_lines(L, plan, False)
+    return axes.value

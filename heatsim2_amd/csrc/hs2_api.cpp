@@ -7,14 +7,17 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <new>
 #include <string>
 #include <tuple>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/heatsim2_amd.h"
 #include "hs2_adjoint.h"
 #include "hs2_batch.h"
 #include "hs2_launch.h"
+#include "hs2_lines.h"
 
 namespace {
 thread_local std::string g_last_error;
@@ -57,6 +60,11 @@ struct hs2_plan {
   bool use_comb = true;         // hs2_plan_set_option(HS2_OPT_COMBINED_X)
   uint8_t *d_comb = nullptr;    // n combined ids
   double *d_ctab = nullptr;     // 12 doubles per id
+  // line tables (class mode): the axes whose distinct lines are factored
+  bool use_lines = true;        // hs2_plan_set_option(HS2_OPT_LINE_TABLES)
+  hs2::RowTab rows{};           // x; g = 0: none
+  hs2::ColTab cols[2] = {};     // [0] z, [1] y; P = 0: none
+  std::vector<void *> d_lines;  // their device arrays
   hs2::DenseView dv{};
   hs2::AsymView av{};
   int ncls[3] = {0, 0, 0};
@@ -198,6 +206,8 @@ hs2::Grid grid_of(const hs2_plan *p) { return hs2::Grid{p->grid.nz, p->grid.ny, 
 hipError_t sweep_x(const hs2_plan *p, const double *Tn, double *Ts, const uint8_t *vmap,
                    const double *vtab, const double *sfield, hipStream_t s, bool ry = false) {
   const hs2::Grid g = grid_of(p);
+  if (p->use_lines && p->rows.g) 
+    return hs2::launch_rows(g, p->rows, Tn, Ts, vmap, vtab, sfield, ry, s);
   if (p->mode == MODE_CLASS && p->have_comb && p->use_comb && !vmap && !sfield &&
       hs2::x_ry_ok(p->xcfg, g))
     return hs2::launch_sweep_x(p->xcfg, g, p->comb, Tn, Ts, s, ry);
@@ -213,6 +223,8 @@ hipError_t sweep_s(const hs2_plan *p, int axis, const double *Tn, const double *
   const hs2::SConfig c = p->scfg[axis];
   const hs2::Grid g = grid_of(p);
   const double dz = p->grid.dz;
+  if (p->use_lines && p->cols[axis].P)
+    return hs2::launch_cols(g, p->cols[axis], axis, Tn, Y, X, surf, dz, ry, s);
   if (p->mode == MODE_CLASS)
     return hs2::launch_sweep_strided(c, g, p->cv, axis, Tn, Y, X, surf, dz, s, ry);
   if (p->mode == MODE_ASYM)
@@ -221,8 +233,9 @@ hipError_t sweep_s(const hs2_plan *p, int axis, const double *Tn, const double *
 }
 
 // the x sweep hands the y sweep its right-hand side instead of T* (one field
-// read less) where the plan and the step allow it
+// read less) where the plan and the step allow it (on line tables always)
 bool use_ry(const hs2_plan *p, bool src) {
+  if (p->use_lines && p->rows.g) return true;
   return p->mode == MODE_CLASS && !src && hs2::x_ry_ok(p->xcfg, grid_of(p));
 }
 
@@ -271,6 +284,13 @@ int source_schedule(int nsteps, const int32_t *h_src_step, int nsrc, const doubl
   return HS2_OK;
 }
 
+void free_lines(hs2_plan *p) {
+  for (void *d : p->d_lines) (void)hipFree(d);
+  p->d_lines.clear();
+  p->rows = hs2::RowTab{};
+  p->cols[0] = p->cols[1] = hs2::ColTab{};
+}
+
 void free_coefficients(hs2_plan *p) {
   (void)hipFree(p->d_cls);
   (void)hipFree(p->d_tab);
@@ -287,6 +307,7 @@ void free_coefficients(hs2_plan *p) {
   p->d_comb = nullptr;
   p->d_ctab = nullptr;
   p->have_comb = false;
+  free_lines(p);
   p->mode = MODE_NONE;
 }
 
@@ -508,6 +529,217 @@ int build_combined(hs2_plan *p, const std::vector<double> &tabs, const int off[4
   return done(HS2_OK);
 }
 
+// Device copy of `v`, owned by the plan's line tables.
+template <class T>
+hipError_t keep_lines(hs2_plan *p, const std::vector<T> &v, const T **out) {
+  void *d = nullptr;
+  hipError_t e = hipMalloc(&d, sizeof(T) * std::max<size_t>(v.size(), 1));
+  if (e != hipSuccess) return e;
+  p->d_lines.push_back(d);
+  *out = static_cast<const T *>(d);
+  return v.empty() ? hipSuccess
+                   : hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+}
+
+// Numbers the distinct lines of one kind (launch_line_hash's `which`):
+// id[line], and the bytes of each distinct line.  *count = 0 where they
+// exceed `most` (or two different lines share a hash): no table then.
+hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
+                          std::vector<int> *id, std::vector<int> *first,
+                          std::vector<uint8_t> *bytes, int *count) {
+  const hs2::Grid g = grid_of(p);
+  const uint8_t *cz = p->cv.cls[0], *cy = p->cv.cls[1], *cx = p->cv.cls[2];
+  unsigned long long *d_hash = nullptr;
+  int *d_rep = nullptr;
+  uint8_t *d_bytes = nullptr;
+  *count = 0;
+  std::vector<unsigned long long> h(2 * (size_t)lines);
+  auto run = [&]() -> hipError_t {
+    hipError_t e = hipMalloc(&d_hash, sizeof(h[0]) * h.size());
+    if (e == hipSuccess) e = hs2::launch_line_hash(g, cz, cy, cx, which, d_hash, 0);
+    if (e == hipSuccess)
+      e = hipMemcpy(h.data(), d_hash, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return e;
+    struct Key {
+      unsigned long long a, b;
+      bool operator==(const Key &o) const { return a == o.a && b == o.b; }
+    };
+    struct Hash {
+      size_t operator()(const Key &k) const { return (size_t)(k.a ^ (k.b >> 7)); }
+    };
+    std::unordered_map<Key, int, Hash> seen;
+    id->assign(lines, 0);
+    first->clear();
+    std::vector<int> rep(lines);
+    for (int ln = 0; ln < lines; ln++) {
+      const Key k{h[2 * (size_t)ln], h[2 * (size_t)ln + 1]};
+      int i;
+      if (ln > 0 && k == Key{h[2 * (size_t)ln - 2], h[2 * (size_t)ln - 1]}) {
+        i = (*id)[ln - 1];
+      } else {
+        auto it = seen.find(k);
+        if (it == seen.end()) {
+          if ((int)first->size() == most) return hipSuccess;
+          it = seen.emplace(k, (int)first->size()).first;
+          first->push_back(ln);
+        }
+        i = it->second;
+      }
+      (*id)[ln] = i;
+      rep[ln] = (*first)[i];
+    }
+    const int cnt = (int)first->size();
+    bytes->resize((size_t)cnt * len);
+    int flag = 0;
+    if ((e = hipMalloc(&d_rep, sizeof(int) * ((size_t)lines + cnt + 1))) != hipSuccess) return e;
+    int *d_first = d_rep + lines, *d_flag = d_first + cnt;
+    if ((e = hipMemcpy(d_rep, rep.data(), sizeof(int) * lines, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(d_first, first->data(), sizeof(int) * cnt, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(d_flag, &flag, sizeof flag, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMalloc(&d_bytes, bytes->size())) != hipSuccess ||
+        (e = hs2::launch_line_check(g, cz, cy, cx, which, d_rep, d_flag, 0)) != hipSuccess ||
+        (e = hs2::launch_line_gather(g, cz, cy, cx, which, d_first, cnt, d_bytes, 0)) != hipSuccess ||
+        (e = hipMemcpy(&flag, d_flag, sizeof flag, hipMemcpyDeviceToHost)) != hipSuccess ||
+        (e = hipMemcpy(bytes->data(), d_bytes, bytes->size(), hipMemcpyDeviceToHost)) != hipSuccess)
+      return e;
+    if (!flag) *count = cnt;
+    return hipSuccess;
+  };
+  const hipError_t e = run();
+  (void)hipFree(d_hash);
+  (void)hipFree(d_rep);
+  (void)hipFree(d_bytes);
+  return e;
+}
+
+// Line tables of the plan's axes (hs2_lines.h), where they pay:
+//   kMostBytes   the distinct lines' factors of an axis: they are read by every
+//                block, beside the field, from an XCD's 4 MB of L2;
+//   kMostGroups  groups of 16 like columns over what 16 columns each would
+//                make (128 x 256 x 256, thin spots at random: z 32.1 us at
+//                1.1, 35.1 at 1.25 and 37.1 at 1.5 against 35.5 for the class
+//                kernel);
+//   kMostVarying the share of rows whose explicit numbers vary along them,
+//                kMostCells the bytes of those numbers (61 x 149 x 203: x
+//                12.6 us without such rows, 17.8 with them all around, 21.6
+//                with them in two planes of three, against 25.8).
+hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int off[4]) {
+  constexpr size_t kMostBytes = size_t(1) << 20, kMostCells = size_t(32) << 20;
+  constexpr double kMostGroups = 1.35, kMostVarying = 0.5;
+  constexpr size_t kRowLds = 32768;  // of the rows' factors in LDS: four blocks per CU
+  const hs2::Grid g = grid_of(p);
+  if ((size_t)p->n * sizeof(double) >= (size_t(1) << 32)) return hipSuccess;
+  std::vector<int> id, first, idx;
+  std::vector<uint16_t> pid;
+  std::vector<uint8_t> bytes;
+  hipError_t e = hipSuccess;
+  int count = 0;
+  auto entry = [&](int axis, uint8_t c) { return &tabs[off[axis] + (size_t)c * hs2::kTabStride]; };
+  for (int axis = 0; axis < 2; axis++) {
+    const int L = axis == 1 ? g.ny : g.nz, ncol = g.nx * (axis == 1 ? g.nz : g.ny);
+    hs2::ColTab t{};
+    hs2::col_shape(L, &t.seg, &t.P);
+    if (!t.P) continue;
+    const size_t per = (size_t)t.P * t.seg * hs2::kColCoef, red = (size_t)t.P * t.P * 4;
+    const int most = (int)std::min<size_t>(65535, kMostBytes / (sizeof(double) * (per + red)));
+    if ((e = distinct_lines(p, axis, ncol, L, most, &id, &first, &bytes, &count)) != hipSuccess)
+      return e;
+    if (!count) continue;
+    auto cell0 = [&](int c) { return axis == 1 ? c / g.nx * g.ny * g.nx + c % g.nx : c; };
+    t.groups = hs2::group_columns(ncol, id, cell0, &idx, &pid);
+    bool ordered = true;  // every group already is 16 neighbours of one line
+    for (int c = 0; c < ncol && ordered; c++) ordered = idx[c] == cell0(c);
+    if (t.groups > kMostGroups * ((ncol + 15) / 16)) continue;
+    std::vector<double> coef(per * count), rd(red * count), M(L), w(L), gm(L);
+    for (int c = 0; c < count; c++) {
+      for (int q = 0; q < L; q++) {
+        const double *v = entry(axis, bytes[(size_t)c * L + q]);
+        M[q] = v[0];
+        w[q] = v[1];
+        gm[q] = v[2];
+      }
+      hs2::factor_column(L, t.seg, t.P, M.data(), w.data(), gm.data(), &coef[per * c],
+                         &rd[red * c], &t.band);
+    }
+    if ((e = keep_lines(p, coef, &t.coef)) != hipSuccess ||
+        (e = keep_lines(p, rd, &t.red)) != hipSuccess ||
+        (!ordered && (e = keep_lines(p, idx, &t.base)) != hipSuccess) ||
+        (e = keep_lines(p, pid, &t.pid)) != hipSuccess)
+      return e;
+    p->cols[axis] = t;
+  }
+  hs2::RowTab t{};
+  int rg = 0;
+  hs2::row_shape(g.nx, &t.cpl, &rg);
+  if (!rg) return hipSuccess;
+  const int nrow = g.nz * g.ny, nc = 2 * hs2::row_pairs(t.cpl);
+  int most = (int)std::min<size_t>(32767, kMostBytes / (sizeof(double) * rg * nc));
+  if ((e = distinct_lines(p, 2, nrow, g.nx, most, &id, &first, &bytes, &count)) != hipSuccess)
+    return e;
+  if (!count) return hipSuccess;
+  std::vector<double> lane((size_t)count * rg * nc), M(g.nx), w(g.nx), gm(g.nx);
+  for (int c = 0; c < count; c++) {
+    for (int q = 0; q < g.nx; q++) {
+      const double *v = entry(2, bytes[(size_t)c * g.nx + q]);
+      M[q] = v[0];
+      w[q] = v[1];
+      gm[q] = v[2];
+    }
+    hs2::factor_row(g.nx, t.cpl, rg, M.data(), w.data(), gm.data(), &lane[(size_t)c * rg * nc],
+                    &t.scan);
+  }
+  std::vector<uint32_t> rid(id.begin(), id.end());
+  // the rows' explicit parts: uniform rows keep six numbers, varying ones six
+  // per cell
+  const size_t per = (size_t)rg * t.cpl * hs2::kRowExpl;
+  if ((e = distinct_lines(p, 3, nrow, 5 * g.nx, 32767, &id, &first, &bytes, &count)) != hipSuccess)
+    return e;
+  if (!count) return hipSuccess;
+  std::vector<double> row, cell;
+  std::vector<uint32_t> eid(count);
+  for (int c = 0; c < count; c++) {
+    const uint8_t *b = &bytes[(size_t)c * 5 * g.nx];
+    const bool lastj = first[c] % g.ny == g.ny - 1, lastk = first[c] / g.ny == g.nz - 1;
+    std::vector<double> v(per, 0.0);
+    bool same = true;
+    for (int i = 0; i < g.nx; i++) {
+      const double *ex = entry(2, b[i]);
+      double *o = &v[(size_t)i * hs2::kRowExpl];
+      o[0] = ex[0];
+      o[1] = ex[1] * entry(1, b[g.nx + i])[2];
+      o[2] = lastj ? 0.0 : ex[1] * entry(1, b[2 * g.nx + i])[2];
+      o[3] = ex[1] * entry(0, b[3 * g.nx + i])[2];
+      o[4] = lastk ? 0.0 : ex[1] * entry(0, b[4 * g.nx + i])[2];
+      o[5] = ex[1];
+      if (i > 0) same &= std::memcmp(o, &v[0], sizeof(double) * hs2::kRowExpl) == 0;
+    }
+    if (same) {
+      eid[c] = (uint32_t)(row.size() / hs2::kRowExpl);
+      row.insert(row.end(), v.begin(), v.begin() + hs2::kRowExpl);
+    } else {
+      if (sizeof(double) * (cell.size() + per) > kMostCells) return hipSuccess;
+      eid[c] = (uint32_t)(cell.size() / per) | hs2::kRowVaries;
+      cell.insert(cell.end(), v.begin(), v.end());
+    }
+  }
+  int varying = 0;
+  for (int r = 0; r < nrow; r++) {
+    rid[r] |= eid[id[r]] << 16;
+    varying += (eid[id[r]] & hs2::kRowVaries) != 0;
+  }
+  if (varying > nrow * kMostVarying) return hipSuccess;
+  if ((e = keep_lines(p, lane, &t.lane)) != hipSuccess ||
+      (e = keep_lines(p, row, &t.row)) != hipSuccess ||
+      (e = keep_lines(p, cell, &t.cell)) != hipSuccess ||
+      (e = keep_lines(p, rid, &t.pid)) != hipSuccess)
+    return e;
+  t.g = rg;
+  t.nlds = (int)std::min<size_t>(lane.size() / ((size_t)rg * nc),
+                                 kRowLds / (sizeof(double) * rg * nc));
+  p->rows = t;
+  return hipSuccess;
+}
+
 }  // namespace
 
 extern "C" {
@@ -654,7 +886,21 @@ int hs2_plan_set_compact(hs2_plan *p, const uint8_t *d_mat, const uint8_t *d_bz,
     p->cv.tab = p->d_tab;
     for (int t = 0; t < 4; t++) p->cv.off[t] = off[t];
     p->mode = MODE_CLASS;
-    return build_combined(p, tabs, off);
+    if ((rc = build_combined(p, tabs, off)) != HS2_OK) return rc;
+    hipError_t e = hipSuccess;
+    try {
+      e = build_lines(p, tabs, off);
+    } catch (const std::bad_alloc &) {
+      e = hipErrorOutOfMemory;
+    }
+    if (e != hipSuccess) {
+      free_lines(p);
+      // without the memory for tables the plan works without them
+      if (e != hipErrorOutOfMemory)
+        return fail(HS2_E_HIP, "hs2_plan_set_compact: line tables: %s", hipGetErrorString(e));
+      (void)hipGetLastError();
+    }
+    return HS2_OK;
   }
   // more than 256 classes on an axis: per-cell float64 coefficients
   double *d_gtab = nullptr, *d_mtab = nullptr;
@@ -767,6 +1013,7 @@ int hs2_plan_set_config(hs2_plan *p, int x_cpl, int x_lanes, int x_lines, int x_
   p->xcfg = xc;
   p->scfg[1] = yc;
   p->scfg[0] = zc;
+  p->use_lines = false;  // the shapes asked for are the class-map kernels'
   return HS2_OK;
 }
 
@@ -776,8 +1023,26 @@ int hs2_plan_set_option(hs2_plan *p, int option, int value) {
     case HS2_OPT_COMBINED_X:
       p->use_comb = value != 0;
       return HS2_OK;
+    case HS2_OPT_LINE_TABLES:
+      p->use_lines = value != 0;
+      return HS2_OK;
     default:
       return fail(HS2_E_ARG, "hs2_plan_set_option: unknown option %d", option);
+  }
+}
+
+int hs2_plan_get_option(const hs2_plan *p, int option, int *value) {
+  if (!p || !value) return fail(HS2_E_ARG, "hs2_plan_get_option: null argument");
+  switch (option) {
+    case HS2_OPT_COMBINED_X:
+      *value = p->use_comb;
+      return HS2_OK;
+    case HS2_OPT_LINE_TABLES:
+      *value = p->use_lines ? (p->rows.g ? 1 : 0) + (p->cols[1].P ? 2 : 0) + (p->cols[0].P ? 4 : 0)
+                            : 0;
+      return HS2_OK;
+    default:
+      return fail(HS2_E_ARG, "hs2_plan_get_option: unknown option %d", option);
   }
 }
 

@@ -185,6 +185,14 @@ __device__ __forceinline__ double2 buf_load_d2(BufRsrc r, unsigned off) {
 __device__ __forceinline__ double buf_load_d(BufRsrc r, unsigned off) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
+// the same with a scalar byte offset besides the lane's
+__device__ __forceinline__ double buf_load_ds(BufRsrc r, unsigned off, unsigned soff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+}
+__device__ __forceinline__ void buf_store_ds(double v, BufRsrc r, unsigned off, unsigned soff) {
+  __builtin_amdgcn_raw_buffer_store_b64(
+      __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, off, soff, 0);
+}
 __device__ __forceinline__ uint32_t buf_load_u32(BufRsrc r, unsigned off) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
 }

@@ -16,7 +16,7 @@
         bytes per launch and in total
 
 Kernels are attributed to sweeps by name (the strided kernel's third
-template argument is its axis).  The last line of the traffic
+template argument is its axis, the line-table kernel's its second).  The last line of the traffic
 summary is ``json: {...}`` with the per-sweep traffic in bytes; bench.py
 reads it.
 """
@@ -54,15 +54,18 @@ def short_name(name):
 
 
 _STRIDED = re.compile(r"k_sweep_strided<[^,<>]+,\s*\d+,\s*(\d+)")
-_STRIDED_RY = re.compile(r"k_sweep_strided<[^,<>]+,\s*\d+,\s*1,\s*(?:true|false),\s*true>")
+_STRIDED_RY = re.compile(r"k_sweep_strided<[^,<>]+,\s*\d+,\s*1,\s*(?:true|false),\s*true>|"
+                         r"k_cols<\d+,\s*1,\s*true,")
+_COLS = re.compile(r"k_cols<\d+,\s*(\d+)")
 
 
 def sweep_of(name):
     """'x', 'y' or 'z' for a sweep kernel's name, else None.  The strided
-    kernel carries its axis (1: y, 0: z) as its third template argument."""
-    if "k_sweep_x" in name:
+    kernel carries its axis (1: y, 0: z) as its third template argument, the
+    line-table one as its second."""
+    if "k_sweep_x" in name or "k_rows" in name:
         return "x"
-    m = _STRIDED.search(name)
+    m = _STRIDED.search(name) or _COLS.search(name)
     if m:
         return "y" if m.group(1) == "1" else "z"
     return None

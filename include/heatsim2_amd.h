@@ -122,9 +122,18 @@ int hs2_plan_set_config(hs2_plan *plan, int x_cpl, int x_lanes, int x_lines, int
  *     source-free steps read one combined class byte per cell (the id of
  *     the cell's z, y, x class triple, built by hs2_plan_set_compact when
  *     there are 256 triples or fewer) instead of the three class planes;
- *     0 reads the three planes.  Same numbers either way. */
-enum { HS2_OPT_COMBINED_X = 1 };
+ *     0 reads the three planes.  Same numbers either way.
+ *   HS2_OPT_LINE_TABLES (default 1; hs2_plan_set_config sets it to 0, since
+ *     its shapes are the other kernels'): with class maps, sweep the axes
+ *     whose lines fall into few distinct ones with those lines' factors,
+ *     computed once by hs2_plan_set_compact; 0 eliminates every line from
+ *     its class bytes on every step.  Same steps to round-off. */
+enum { HS2_OPT_COMBINED_X = 1, HS2_OPT_LINE_TABLES = 2 };
 int hs2_plan_set_option(hs2_plan *plan, int option, int value);
+
+/* An option's value; for HS2_OPT_LINE_TABLES the axes that are swept so
+ * (1 x, 2 y, 4 z, added up; 0 when off). */
+int hs2_plan_get_option(const hs2_plan *plan, int option, int *value);
 
 /* info[0..13] = mode (0 none, 1 class maps, 2 dense, 3 dense per side),
  * classes per axis z/y/x, x_cpl, x_lanes, y_seg, y_lines, z_seg, z_lines,
