@@ -4,6 +4,7 @@
 #include <functional>
 #include <vector>
 
+#include "hs2_dense.h"
 #include "hs2_lines.h"
 
 namespace hs2 {
@@ -135,18 +136,20 @@ __global__ __launch_bounds__(512) void k_cols(Grid g, ColTab t, int cs, const do
   const BufRsrc bT = make_buf(Tn, bytes), bY = make_buf(Y, bytes), bX = make_buf(X, bytes);
   const unsigned so = (unsigned)stride * 8u, vo = (unsigned)base * 8u + (unsigned)t0 * so;
   // Rows past the line's end read what follows it in the array, or 0 past the
-  // array's end (the buffer's bound); they are cleared below.
+  // array's end (the buffer's bound, which holds for the lane's offset but not
+  // for a scalar one: the row offset is added to the former); they are cleared
+  // below.
   double d[SEG + 1], y[SEG];  // differences of T^n across the rows' faces
   if constexpr (!RY) {
     double T[SEG + 2];
-    T[0] = buf_load_ds(bT, t0 > 0 ? vo - so : vo, 0);
+    T[0] = buf_load_d(bT, t0 > 0 ? vo - so : vo);
 #pragma unroll
-    for (int q = 0; q <= SEG; q++) T[q + 1] = buf_load_ds(bT, vo, q * so);
+    for (int q = 0; q <= SEG; q++) T[q + 1] = buf_load_d(bT, vo + q * so);
 #pragma unroll
     for (int q = 0; q <= SEG; q++) d[q] = T[q + 1] - T[q];
   }
 #pragma unroll
-  for (int q = 0; q < SEG; q++) y[q] = buf_load_ds(bY, vo, q * so);
+  for (int q = 0; q < SEG; q++) y[q] = buf_load_d(bY, vo + q * so);
   const bool whole = t0 + SEG <= L;
   if (t0 + SEG >= L) {
     if constexpr (!RY) {
@@ -216,43 +219,6 @@ __global__ __launch_bounds__(512) void k_cols(Grid g, ColTab t, int cs, const do
 }
 
 // --------------------------------------------------------------- rows
-// 16-byte accesses to cells whose row may start on any cell: 8-byte alignment
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
-
-template <int CPL>
-__device__ __forceinline__ void load_cells(const double *__restrict__ a, int idx, int n,
-                                           double (&v)[CPL]) {
-  if (idx + CPL <= n) {
-#pragma unroll
-    for (int q = 0; q + 1 < CPL; q += 2) {
-      const d2u d = *reinterpret_cast<const d2u *>(a + idx + q);
-      v[q] = d.x;
-      v[q + 1] = d.y;
-    }
-    if (CPL & 1) v[CPL - 1] = a[idx + CPL - 1];
-  } else {
-#pragma unroll
-    for (int q = 0; q < CPL; q++) v[q] = a[min(idx + q, n - 1)];
-  }
-}
-// the class bytes of up to eight cells, first one lowest
-template <int CPL>
-__device__ __forceinline__ uint64_t load_classes(const uint8_t *__restrict__ a, int idx, int n) {
-  typename std::conditional<(CPL > 4), uint64_t, uint32_t>::type w = 0;
-  if (idx + (int)sizeof w <= n) {
-    __builtin_memcpy(&w, a + idx, sizeof w);
-    return w;
-  }
-  uint64_t v = 0;
-#pragma unroll
-  for (int q = 0; q < CPL; q++) v |= (uint64_t)a[min(idx + q, n - 1)] << (8 * q);
-  return v;
-}
-
-// lane l of the wave reads lane l-1 (up) or l+1 (down); 0 at the wave's ends
-__device__ __forceinline__ double wave_up(double v) { return dpp_d<0x138>(v); }
-__device__ __forceinline__ double wave_down(double v) { return dpp_d<0x130>(v); }
-
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp_rows(double v) {
   const long long b = __double_as_longlong(v);
@@ -388,7 +354,7 @@ __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__
     [[maybe_unused]] uint64_t cls = 0;
     [[maybe_unused]] double S[CPL] = {};
     if constexpr (SRC) {
-      if (vmap) cls = load_classes<CPL>(vmap, (k * ny + j) * nx + ir, n);
+      if (vmap) cls = load_bytes<CPL>(vmap, (k * ny + j) * nx + ir, n);
       if (sfield) load_cells<CPL>(sfield, (k * ny + j) * nx + ir, n, S);
     }
     double TL = wave_up(T[CPL - 1]), TR = wave_down(T[0]);
