@@ -32,6 +32,9 @@ X_COMBOS = ((1, 16, 0), (2, 16, 0), (4, 16, 0), (8, 16, 0), (16, 16, 0), (2, 32,
 SEGS = (2, 4, 8, 16, 32)
 LINES = (8, 16, 32, 64)
 MAX_BLOCK = 512
+# Per-voxel coefficients (plan modes 2 and 3) have fixed shapes up to these
+# axis lengths: nothing to choose there.
+DENSE_X, DENSE_YZ = 256, 512
 
 _memo = {}
 
@@ -123,9 +126,12 @@ def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
            "y": (info["y_seg"], info["y_lines"]),
            "z": (info["z_seg"], info["z_lines"])}
     best_ms = [None, None, None]
+    dense = info["mode"] in (2, 3)
     for axis_name, idx, cands in (("x", 0, x_candidates(nx)), ("y", 1, strided_candidates(ny)),
                                   ("z", 2, strided_candidates(nz))):
         results = []
+        if dense and (nx <= DENSE_X if axis_name == "x" else (nz, ny)[idx == 1] <= DENSE_YZ):
+            cands = [cur[axis_name]]
         for cand in cands:
             trial = dict(cur)
             trial[axis_name] = cand

@@ -30,6 +30,7 @@
 
 #include "hs2_adjoint.h"
 #include "hs2_batch.h"
+#include "hs2_launch.h"
 
 namespace hs2 {
 
@@ -39,38 +40,21 @@ namespace hs2 {
 // Axes 1, 0: columns i = bx*CW + cl, by = k (y) or j (z).  A block has P
 // thread segments of SEG cells per line; P = blockDim.x / CW.  U must not
 // alias R.
-// FLAT (batched, axes 0 and 1): columns as in sweep_strided_body's FLAT, by
-// = P segments per line.
-template <class V, int SEG, int AXIS, bool FLAT = false>
+template <class V, int SEG, int AXIS>
 __device__ __forceinline__ void adj_line_body(Grid g, V view, int CW, const double *R,
                                               int scale_m, double *U, int bx, int by) {
-  static_assert(!(FLAT && AXIS == 2), "x lines are not flattened");
   extern __shared__ double lds[];
   view.load_tables(lds, AXIS);
-  const int P = FLAT ? by : blockDim.x / CW;
+  const int P = blockDim.x / CW;
   double *ra = lds + ((view.lds_doubles(AXIS) + 1) & ~1);
   double *rc = ra + 2 * P * CW;
   double *rr = rc + 2 * P * CW;
   __syncthreads();
 
   const int cl = threadIdx.x % CW, p = threadIdx.x / CW;
-  const bool act = !FLAT || p < P;
   int L, stride, base;
   bool valid;
-  if constexpr (FLAT) {
-    L = AXIS == 1 ? g.ny : g.nz;
-    stride = AXIS == 1 ? g.nx : g.nx * g.ny;
-    const int ncol = g.nx * (AXIS == 1 ? g.nz : g.ny);
-    const int col = bx * CW + cl;
-    valid = act && col < ncol;
-    const int cc = min(col, ncol - 1);
-    if (AXIS == 1) {
-      const int k = cc / g.nx;
-      base = k * g.ny * g.nx + (cc - k * g.nx);
-    } else {
-      base = cc;
-    }
-  } else if (AXIS == 2) {
+  if (AXIS == 2) {
     const int nl = g.nz * g.ny, line = bx * CW + cl;
     valid = line < nl;
     L = g.nx;
@@ -116,12 +100,10 @@ __device__ __forceinline__ void adj_line_body(Grid g, V view, int CW, const doub
   }
   double As, Cs, Rs, Ae, Ce, Re;
   segment_reduce<SEG>(a, c, r, As, Cs, Rs, Ae, Ce, Re);
-  if (act) {
-    ra[(2 * p) * CW + cl] = As; rc[(2 * p) * CW + cl] = Cs; rr[(2 * p) * CW + cl] = Rs;
-    ra[(2 * p + 1) * CW + cl] = Ae; rc[(2 * p + 1) * CW + cl] = Ce; rr[(2 * p + 1) * CW + cl] = Re;
-  }
+  ra[(2 * p) * CW + cl] = As; rc[(2 * p) * CW + cl] = Cs; rr[(2 * p) * CW + cl] = Rs;
+  ra[(2 * p + 1) * CW + cl] = Ae; rc[(2 * p + 1) * CW + cl] = Ce; rr[(2 * p + 1) * CW + cl] = Re;
   __syncthreads();
-  lds_pcr_ends(ra, rc, rr, p, P, CW, cl, act);
+  lds_pcr_ends(ra, rc, rr, p, P, CW, cl);
   if (!valid) return;
   const double xs = rr[(2 * p) * CW + cl], xe = rr[(2 * p + 1) * CW + cl];
   double x[SEG];
@@ -133,100 +115,6 @@ __device__ __forceinline__ void adj_line_body(Grid g, V view, int CW, const doub
   for (int q = 0; q < SEG; q++) {
     const int t = t0 + q;
     if (t < L) U[base + t * stride] = x[q];
-  }
-}
-
-// adj_line_body for x lines of per-voxel coefficients, staged through LDS:
-// the block's CW x-lines are consecutive in memory, so the right-hand side is
-// loaded cell by cell along the lines (coalesced) into padded LDS rows, and
-// the solution leaves through LDS the same way; each thread reads its
-// segment's x entries (M, g, w) from memory itself (staging them as well
-// quadrupled the block's LDS and cost more in occupancy than the strided
-// loads do).  LDS: 6 P CW doubles of reduced rows, then CW rows of (L | 1)
-// doubles.
-template <int SEG>
-__device__ __forceinline__ void adj_x_staged_body(Grid g, DenseView view, int CW, const double *R,
-                                                  int scale_m, double *U, int bx) {
-  extern __shared__ double lds[];
-  const int P = blockDim.x / CW;
-  const int L = g.nx, RW = g.nx | 1;
-  double *ra = lds;
-  double *rc = ra + 2 * P * CW;
-  double *rr = rc + 2 * P * CW;
-  double *sR = rr + 2 * P * CW;
-  const int nl = g.nz * g.ny, l0 = bx * CW;
-  const int nlb = min(CW, nl - l0);
-  const int ncell = nlb * L;
-  const long long c0 = (long long)l0 * L;
-  // UN cells per thread per batch, all loads issued before the first use
-  constexpr int UN = 8;
-  for (int e0 = 0; e0 < ncell; e0 += UN * (int)blockDim.x) {
-    double vr[UN];
-#pragma unroll
-    for (int u = 0; u < UN; u++) {
-      const long long c = c0 + min(e0 + u * (int)blockDim.x + (int)threadIdx.x, ncell - 1);
-      vr[u] = R[c];
-    }
-#pragma unroll
-    for (int u = 0; u < UN; u++) {
-      const int e = e0 + u * (int)blockDim.x + (int)threadIdx.x;
-      if (e < ncell) {
-        const int lc = e / L;
-        sR[lc * RW + (e - lc * L)] = vr[u];
-      }
-    }
-  }
-  __syncthreads();
-  const int cl = threadIdx.x % CW, p = threadIdx.x / CW;
-  const bool valid = cl < nlb;
-  const int row = (valid ? cl : 0) * RW;
-  const long long grow = c0 + (long long)(valid ? cl : 0) * L;
-  const int t0 = p * SEG;
-  auto entry = [&](int t) {
-    const long long o = grow + min(max(t, 0), L - 1);
-    return Entry{view.M[o], (double)view.w[o], view.g[2][o]};
-  };
-  double a[SEG], c[SEG], r[SEG];
-  Entry em = entry(t0 - 1);
-  Entry ec = entry(t0);
-#pragma unroll
-  for (int q = 0; q < SEG; q++) {
-    const int t = t0 + q;
-    const Entry ep = entry(t + 1);
-    const double gm = t >= 1 ? ec.g : 0.0;
-    const double gp = t + 1 <= L - 1 ? ep.g : 0.0;
-    const double b = ec.M + 0.5 * ec.w * (gm + gp);
-    const double inv = 1.0 / b;
-    const double Rq = sR[row + min(t, L - 1)];
-    const double rhs = scale_m ? ec.M * Rq : Rq;
-    const bool ok = valid && t < L;
-    a[q] = ok ? -0.5 * em.w * gm * inv : 0.0;
-    c[q] = ok ? -0.5 * ep.w * gp * inv : 0.0;
-    r[q] = ok ? rhs * inv : 0.0;
-    em = ec;
-    ec = ep;
-  }
-  double As, Cs, Rs, Ae, Ce, Re;
-  segment_reduce<SEG>(a, c, r, As, Cs, Rs, Ae, Ce, Re);
-  ra[(2 * p) * CW + cl] = As; rc[(2 * p) * CW + cl] = Cs; rr[(2 * p) * CW + cl] = Rs;
-  ra[(2 * p + 1) * CW + cl] = Ae; rc[(2 * p + 1) * CW + cl] = Ce; rr[(2 * p + 1) * CW + cl] = Re;
-  __syncthreads();
-  // (every thread has built its rows from sR before the barriers in here,
-  // so sR can take the solution afterwards)
-  lds_pcr_ends(ra, rc, rr, p, P, CW, cl);
-  const double xs = rr[(2 * p) * CW + cl], xe = rr[(2 * p + 1) * CW + cl];
-  if (valid) {
-#pragma unroll
-    for (int q = 0; q < SEG; q++) {
-      const int t = t0 + q;
-      const double x = q == 0 ? xs : q == SEG - 1 ? xe : r[q] - a[q] * xs - c[q] * xe;
-      if (t < L) sR[row + t] = x;
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < ncell; e += blockDim.x) {
-    const int lc = e / L;
-    U[c0 + e] = sR[lc * RW + (e - lc * L)];
   }
 }
 
@@ -393,6 +281,8 @@ hipError_t launch_adj_line(const Grid &g, const ClassView &v, int axis, const do
 }
 hipError_t launch_adj_line(const Grid &g, const DenseView &v, int axis, const double *R,
                            int scale_m, double *U, hipStream_t s) {
+  if (axis == 2 ? dense_rows_ok(g) : dense_cols_ok(g, axis))
+    return launch_dense_adj(g, v, axis, R, scale_m, U, s);
   return launch_adj_line_v(g, v, axis, R, scale_m, U, s);
 }
 
@@ -429,23 +319,6 @@ hipError_t launch_fill(double *a, size_t n, double v, hipStream_t s) {
 
 
 // ------------------------------------------------------ batched adjoint
-template <int SEG, int AXIS>
-__global__ __launch_bounds__(kBatchThreads) void kb_adj_line(BatchMap m, DenseView v,
-                                                             const double *R, int scale_m,
-                                                             double *U) {
-  BatchInst I;
-  int local, t;
-  if (!batch_locate(m, I, local, t)) return;
-  const int cw = I.cw[AXIS];
-  if constexpr (AXIS == 2)
-    adj_x_staged_body<SEG>(Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off), cw, R + I.off, scale_m,
-                           U + I.off, local);
-  else
-    adj_line_body<DenseView, SEG, AXIS, true>(Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off), cw,
-                                              R + I.off, scale_m, U + I.off, local,
-                                              batch_line_segs(AXIS == 1 ? I.ny : I.nz));
-}
-
 // f: base pointers of the concatenated fields; f.ghist: base of the
 // concatenated dJ/dhist; f.gsrc: base of the concatenated source gradients.
 __global__ __launch_bounds__(256) void kb_adj_stencil(BatchMap m, DenseView v, AdjFields f) {
@@ -493,22 +366,6 @@ __global__ void kb_lam_init(BatchMap m, const double *ghist, double *lam) {
 // ctr[which] = value (set) or += value (add); one thread
 __global__ void kb_counter(int *ctr, int which, int value, int add) {
   if (threadIdx.x == 0 && blockIdx.x == 0) ctr[which] = add ? ctr[which] + value : value;
-}
-
-hipError_t launch_batch_adj_line(const BatchMap &m, int nblocks, int axis, const DenseView &v,
-                                 const double *R, int scale_m, double *U, hipStream_t s) {
-  // x lines: blocks of kBatchXThreads staging CW rows of (L | 1) right-hand
-  // sides, CW L <= kBatchXThreads kBatchSeg
-  const int threads = axis == 2 ? kBatchXThreads : kBatchThreads;
-  const size_t rows = (size_t)kBatchXThreads * kBatchSeg + kBatchXThreads;
-  const size_t shm = sizeof(double) * (6 * (size_t)threads + (axis == 2 ? rows : 0));
-  const dim3 grid(nblocks), block(threads);
-  switch (axis) {
-    case 0: hipLaunchKernelGGL((kb_adj_line<kBatchSeg, 0>), grid, block, shm, s, m, v, R, scale_m, U); break;
-    case 1: hipLaunchKernelGGL((kb_adj_line<kBatchSeg, 1>), grid, block, shm, s, m, v, R, scale_m, U); break;
-    default: hipLaunchKernelGGL((kb_adj_line<kBatchSeg, 2>), grid, block, shm, s, m, v, R, scale_m, U); break;
-  }
-  return hipGetLastError();
 }
 
 hipError_t launch_batch_adj_stencil(const BatchMap &m, int nblocks, const DenseView &v,

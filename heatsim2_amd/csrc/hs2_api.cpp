@@ -214,8 +214,8 @@ hipError_t sweep_x(const hs2_plan *p, const double *Tn, double *Ts, const uint8_
   if (p->mode == MODE_CLASS)
     return hs2::launch_sweep_x(p->xcfg, g, p->cv, Tn, Ts, vmap, vtab, sfield, s, ry);
   if (p->mode == MODE_ASYM)
-    return hs2::launch_sweep_x(p->xcfg, g, p->av, Tn, Ts, vmap, vtab, sfield, s);
-  return hs2::launch_sweep_x(p->xcfg, g, p->dv, Tn, Ts, vmap, vtab, sfield, s);
+    return hs2::launch_sweep_x(p->xcfg, g, p->av, Tn, Ts, vmap, vtab, sfield, s, ry);
+  return hs2::launch_sweep_x(p->xcfg, g, p->dv, Tn, Ts, vmap, vtab, sfield, s, ry);
 }
 
 hipError_t sweep_s(const hs2_plan *p, int axis, const double *Tn, const double *Y, double *X,
@@ -228,14 +228,16 @@ hipError_t sweep_s(const hs2_plan *p, int axis, const double *Tn, const double *
   if (p->mode == MODE_CLASS)
     return hs2::launch_sweep_strided(c, g, p->cv, axis, Tn, Y, X, surf, dz, s, ry);
   if (p->mode == MODE_ASYM)
-    return hs2::launch_sweep_strided(c, g, p->av, axis, Tn, Y, X, surf, dz, s);
-  return hs2::launch_sweep_strided(c, g, p->dv, axis, Tn, Y, X, surf, dz, s);
+    return hs2::launch_sweep_strided(c, g, p->av, axis, Tn, Y, X, surf, dz, s, ry);
+  return hs2::launch_sweep_strided(c, g, p->dv, axis, Tn, Y, X, surf, dz, s, ry);
 }
 
 // the x sweep hands the y sweep its right-hand side instead of T* (one field
-// read less) where the plan and the step allow it (on line tables always)
+// read less) where the plan and the step allow it (on line tables always, on
+// per-voxel coefficients by the grid)
 bool use_ry(const hs2_plan *p, bool src) {
   if (p->use_lines && p->rows.g) return true;
+  if (p->mode == MODE_DENSE || p->mode == MODE_ASYM) return hs2::dense_ry(grid_of(p));
   return p->mode == MODE_CLASS && !src && hs2::x_ry_ok(p->xcfg, grid_of(p));
 }
 
@@ -322,10 +324,10 @@ hs2::BatchMap batch_map(const hs2_batch *b, int kind, int rule, int j) {
 
 int blocks_of(const hs2::BatchInst &I, int kind) {
   switch (kind) {
-    case KIND_X2: return (I.nz * I.ny + hs2::kBatchXLines - 1) / hs2::kBatchXLines;
+    case KIND_X2: return (I.units + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
     case KIND_Y: return (I.nx * I.nz + I.cw[1] - 1) / I.cw[1];
     case KIND_Z: return (I.nx * I.ny + I.cw[0] - 1) / I.cw[0];
-    case KIND_AX: return (I.nz * I.ny + I.cw[2] - 1) / I.cw[2];
+    case KIND_AX: return (I.rows + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
     default: return (int)(((long long)I.nz * I.ny * I.nx + 255) / 256);
   }
 }
@@ -369,14 +371,14 @@ hipError_t emit_forward(hs2_batch *b, double *T, const double *src, double *hist
                         const BatchWork &w, int steps, hipStream_t s) {
   hipError_t e = hipSuccess;
   for (int c = 0; c < steps && e == hipSuccess; c++) {
-    e = hs2::launch_batch_x2(batch_map(b, KIND_X2, hs2::RULE_FWD, 0), b->nblk[KIND_X2], b->dv, T,
-                             w.ws, src, w.ck, s);
+    e = hs2::launch_batch_rows(batch_map(b, KIND_X2, hs2::RULE_FWD, 0), b->nblk[KIND_X2], b->dv,
+                               T, w.ws, src, w.ck, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_strided(batch_map(b, KIND_Y, hs2::RULE_FWD, 0), b->nblk[KIND_Y], 1,
-                                    b->dv, T, w.ws, w.ws, nullptr, s);
+      e = hs2::launch_batch_cols(batch_map(b, KIND_Y, hs2::RULE_FWD, 0), b->nblk[KIND_Y], 1, b->dv,
+                                 T, w.ws, w.ws, nullptr, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_strided(batch_map(b, KIND_Z, hs2::RULE_FWD, 0), b->nblk[KIND_Z], 0,
-                                    b->dv, T, w.ws, T, hist, s);
+      e = hs2::launch_batch_cols(batch_map(b, KIND_Z, hs2::RULE_FWD, 0), b->nblk[KIND_Z], 0, b->dv,
+                                 T, w.ws, T, hist, false, s);
     if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 0, 1, 1, s);
   }
   return e;
@@ -394,14 +396,14 @@ hipError_t emit_backward_segment(hs2_batch *b, const double *src, const double *
   for (int j = 0; j < K && e == hipSuccess; j++) {
     const double *in = w.seg + (size_t)j * N;
     double *tx = w.segx + (size_t)j * N, *ty = w.segy + (size_t)j * N;
-    e = hs2::launch_batch_x2(batch_map(b, KIND_X2, hs2::RULE_RECOMP, j), b->nblk[KIND_X2], b->dv,
-                             in, tx, src, nullptr, s);
+    e = hs2::launch_batch_rows(batch_map(b, KIND_X2, hs2::RULE_RECOMP, j), b->nblk[KIND_X2], b->dv,
+                               in, tx, src, nullptr, false, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_strided(batch_map(b, KIND_Y, hs2::RULE_RECOMP, j), b->nblk[KIND_Y], 1,
-                                    b->dv, in, tx, ty, nullptr, s);
+      e = hs2::launch_batch_cols(batch_map(b, KIND_Y, hs2::RULE_RECOMP, j), b->nblk[KIND_Y], 1,
+                                 b->dv, in, tx, ty, nullptr, false, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_strided(batch_map(b, KIND_Z, hs2::RULE_RECOMP, j), b->nblk[KIND_Z], 0,
-                                    b->dv, in, ty, w.seg + (size_t)(j + 1) * N, nullptr, s);
+      e = hs2::launch_batch_cols(batch_map(b, KIND_Z, hs2::RULE_RECOMP, j), b->nblk[KIND_Z], 0,
+                                 b->dv, in, ty, w.seg + (size_t)(j + 1) * N, nullptr, false, s);
   }
   // adjoint steps, latest first: z, y, x transposed line solves from
   // lam = dJ/dT^{t+1}, then the stencil, which leaves dJ/dT^t in lam
@@ -1333,10 +1335,12 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
     hs2::BatchInst I{};
     I.nz = s.nz; I.ny = s.ny; I.nx = s.nx; I.nsteps = s.nsteps;
     I.src_step = s.src_step; I.dz = s.dz;
-    I.xseg = hs2::batch_x_seg(s.nx);
+    I.row = hs2::batch_row(s.nx);
+    const int rg = hs2::batch_row_group(s.nx);
+    I.units = (s.ny + rg - 1) / rg * ((s.nz + hs2::kBatchPlanes - 1) / hs2::kBatchPlanes);
+    I.rows = (s.ny * s.nz + rg - 1) / rg;
     I.cw[0] = hs2::batch_flat_cw(s.nz);
     I.cw[1] = hs2::batch_flat_cw(s.ny);
-    I.cw[2] = hs2::batch_line_cw(s.nx, hs2::kBatchXThreads);
     const long long n = (long long)s.nz * s.ny * s.nx;
     I.off = off;
     I.hoff = hoff;

@@ -20,10 +20,10 @@
 namespace hs2 {
 
 constexpr int kBatchMaxLen = 128;  // axis length limit of the batched kernels
-constexpr int kBatchThreads = 256; // threads per block of the strided / line kernels
-constexpr int kBatchXThreads = 128; // threads per block of the adjoint x-line kernel
+constexpr int kBatchThreads = 256; // threads per block of the y and z kernels
+constexpr int kBatchWaves = 4;     // waves (units of rows) per block of the x kernels
 constexpr int kBatchSeg = 8;       // cells per thread segment of the line kernels
-constexpr int kBatchXLines = 8;    // x-lines per block of the batched x sweep (16 lanes each)
+constexpr int kBatchPlanes = 2;    // planes a wave of the x sweep walks (1, 4: 2% slower, 8: 18%)
 constexpr int kBatchAlign = 32;    // instance offsets are multiples of this many cells
 
 // Segments of kBatchSeg cells per line of L cells in the y and z line
@@ -31,15 +31,12 @@ constexpr int kBatchAlign = 32;    // instance offsets are multiples of this man
 // side by side, cw = floor(256 / P): consecutive columns in memory order.
 __host__ __device__ inline int batch_line_segs(int L) { return (L + kBatchSeg - 1) / kBatchSeg; }
 __host__ __device__ inline int batch_flat_cw(int L) { return kBatchThreads / batch_line_segs(L); }
-// Lines per block of the adjoint x-line kernel (threads / a power-of-two
-// count of segments covering L).
-__host__ __device__ inline int batch_line_cw(int L, int threads = kBatchThreads) {
-  int p = 1;
-  while (p * kBatchSeg < L) p <<= 1;
-  return threads / p;
+// The x kernels' row shape by nx: 16 lanes x 2 or 4 cells, 32 x 3 or 4; and the
+// rows a wave holds.
+__host__ __device__ inline int batch_row(int nx) {
+  return nx <= 32 ? 0 : nx <= 64 ? 1 : nx <= 96 ? 2 : 3;
 }
-// cells per lane (16 lanes per line) of the batched x sweep's solve
-__host__ __device__ inline int batch_x_seg(int nx) { return nx <= 32 ? 2 : nx <= 64 ? 4 : 8; }
+__host__ __device__ inline int batch_row_group(int nx) { return nx <= 64 ? 4 : 2; }
 
 struct BatchInst {
   int nz, ny, nx, nsteps;
@@ -47,11 +44,10 @@ struct BatchInst {
   long long hoff;   // first value of the surface history (nsteps x ny x nx)
   long long ckoff;  // first value of the checkpoints (ceil(nsteps/K) fields)
   int src_step;     // step whose source field applies (-1: none)
-  int xseg;         // batch_x_seg(nx)
-  int cw[3];        // lines per block: batch_flat_cw of the z and y line
-                    // lengths, batch_line_cw of x's for the adjoint x-line
-                    // kernel's kBatchXThreads
-  int pad;
+  int row;          // batch_row(nx)
+  int units;        // waves of the x sweep: row groups x chunks of kBatchPlanes planes
+  int rows;         // waves of the adjoint x solve: row groups
+  int cw[2];        // lines per block: batch_flat_cw of the z and y line lengths
   double dz;
 };
 
@@ -122,13 +118,13 @@ __device__ __forceinline__ DenseView offset_view(DenseView v, long long off) {
 namespace hs2 {
 struct AdjFields;
 // launchers (hs2_kernels.hip, hs2_adjoint.hip); nblocks = this kind's block total
-// the x sweep; with ck != nullptr (forward) a block first copies its lines of
-// T^t into the instance's checkpoint slot on a checkpoint step
-hipError_t launch_batch_x2(const BatchMap &m, int nblocks, const DenseView &v, const double *Tn,
-                           double *Ts, const double *src, double *ck, hipStream_t s);
-hipError_t launch_batch_strided(const BatchMap &m, int nblocks, int axis, const DenseView &v,
-                                const double *Tn, const double *Y, double *X, double *hist,
-                                hipStream_t s);
+// the x sweep; with ck != nullptr (forward) T^t is copied into the instance's
+// checkpoint slot on a checkpoint step; ry as for a plan's sweeps
+hipError_t launch_batch_rows(const BatchMap &m, int nblocks, const DenseView &v, const double *Tn,
+                             double *Ts, const double *src, double *ck, bool ry, hipStream_t s);
+hipError_t launch_batch_cols(const BatchMap &m, int nblocks, int axis, const DenseView &v,
+                             const double *Tn, const double *Y, double *X, double *hist, bool ry,
+                             hipStream_t s);
 hipError_t launch_batch_adj_line(const BatchMap &m, int nblocks, int axis, const DenseView &v,
                                  const double *R, int scale_m, double *U, hipStream_t s);
 hipError_t launch_batch_adj_stencil(const BatchMap &m, int nblocks, const DenseView &v,

@@ -723,15 +723,14 @@ __global__ __launch_bounds__(G *LPB) void k_sweep_x2(Grid g, V view,
 // instance's lines taken in memory order (axis 0: the (j, i) plane, axis 1:
 // the (k, i) columns), and by is P, the segments per line; P x CW may fall
 // short of the block, whose remaining threads only take part in barriers.
-template <class V, int SEG, int AXIS, bool FULL = false, bool RY = false, bool FLAT = false>
+template <class V, int SEG, int AXIS, bool FULL = false, bool RY = false>
 __device__ __forceinline__ void sweep_strided_body(Grid g, V view, int CW, const double *Tn,
                                                    const double *Y, double *X, double *surf,
                                                    double dz, int bx, int by) {
   constexpr int axis = AXIS;
-  static_assert(!(FLAT && FULL), "FLAT lines are masked");
   extern __shared__ double lds[];
   view.load_tables(lds, axis);
-  const int P = FLAT ? by : blockDim.x / CW;
+  const int P = blockDim.x / CW;
   double *ra = lds + ((view.lds_doubles(axis) + 1) & ~1);
   double *rc = ra + 2 * P * CW;
   double *rr = rc + 2 * P * CW;
@@ -739,28 +738,12 @@ __device__ __forceinline__ void sweep_strided_body(Grid g, V view, int CW, const
 
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int cl = threadIdx.x % CW, p = threadIdx.x / CW;
-  const bool act = !FLAT || p < P;
   const int L = axis == 1 ? ny : nz;
   const int stride = axis == 1 ? nx : nx * ny;
-  bool valid;
-  int base;
-  if constexpr (FLAT) {
-    const int ncol = nx * (axis == 1 ? nz : ny);
-    const int col = bx * CW + cl;
-    valid = act && col < ncol;
-    const int cc = min(col, ncol - 1);
-    if (axis == 1) {
-      const int k = cc / nx;
-      base = k * ny * nx + (cc - k * nx);
-    } else {
-      base = cc;
-    }
-  } else {
-    const int i = bx * CW + cl;
-    valid = i < nx;
-    const int ic = valid ? i : nx - 1;
-    base = axis == 1 ? by * ny * nx + ic : by * nx + ic;
-  }
+  const int i = bx * CW + cl;
+  const bool valid = i < nx;
+  const int ic = valid ? i : nx - 1;
+  const int base = axis == 1 ? by * ny * nx + ic : by * nx + ic;
   const int t0 = p * SEG;
 
   // ---- loads: T^n over the segment plus one halo cell each side, Y, entries
@@ -829,12 +812,10 @@ __device__ __forceinline__ void sweep_strided_body(Grid g, V view, int CW, const
     segment_reduce_halves<SEG>(a, c, r, As, Cs, Rs, Ae, Ce, Re, hj);
   else
     segment_reduce<SEG>(a, c, r, As, Cs, Rs, Ae, Ce, Re);
-  if (act) {
-    ra[(2 * p) * CW + cl] = As; rc[(2 * p) * CW + cl] = Cs; rr[(2 * p) * CW + cl] = Rs;
-    ra[(2 * p + 1) * CW + cl] = Ae; rc[(2 * p + 1) * CW + cl] = Ce; rr[(2 * p + 1) * CW + cl] = Re;
-  }
+  ra[(2 * p) * CW + cl] = As; rc[(2 * p) * CW + cl] = Cs; rr[(2 * p) * CW + cl] = Rs;
+  ra[(2 * p + 1) * CW + cl] = Ae; rc[(2 * p + 1) * CW + cl] = Ce; rr[(2 * p + 1) * CW + cl] = Re;
   __syncthreads();
-  lds_pcr_ends(ra, rc, rr, p, P, CW, cl, act);
+  lds_pcr_ends(ra, rc, rr, p, P, CW, cl);
   if (!valid) return;
   const double xs = rr[(2 * p) * CW + cl], xe = rr[(2 * p + 1) * CW + cl];
   double x[SEG];
@@ -1016,16 +997,20 @@ static hipError_t launch_x_v(XConfig cfg, const Grid &g, const V &v, const doubl
                              double *Ts, const uint8_t *vmap, const double *vtab,
                              const double *sfield, bool ry, hipStream_t s) {
   if (ry && cfg.lpb == 0) return hipErrorInvalidValue;
+  // per-voxel rows of up to 256 cells never come here (dense_rows_ok)
+  constexpr int kLeast = std::is_same<V, ClassView>::value ? 1 : 257;
 #define HS2_X(C, GG)                                                               \
-  if (cfg.lpb == 0 && cfg.cpl == C && cfg.g == GG)                                 \
-    return launch_x_t<V, C, GG>(g, v, Tn, Ts, vmap, vtab, sfield, s);
+  if constexpr (C * GG >= kLeast)                                                  \
+    if (cfg.lpb == 0 && cfg.cpl == C && cfg.g == GG)                               \
+      return launch_x_t<V, C, GG>(g, v, Tn, Ts, vmap, vtab, sfield, s);
   HS2_X(1, 16) HS2_X(2, 16) HS2_X(4, 16) HS2_X(8, 16) HS2_X(16, 16)
   HS2_X(2, 32) HS2_X(4, 32) HS2_X(8, 32) HS2_X(16, 32)
   HS2_X(2, 64) HS2_X(4, 64) HS2_X(8, 64) HS2_X(16, 64)
 #undef HS2_X
 #define HS2_X2(C, GG, LL)                                                          \
-  if (cfg.lpb == LL && cfg.cpl == C && cfg.g == GG)                                \
-    return launch_x2_t<V, C, GG, LL>(g, v, cfg.ty, Tn, Ts, vmap, vtab, sfield, ry, s);
+  if constexpr (C * GG >= kLeast)                                                  \
+    if (cfg.lpb == LL && cfg.cpl == C && cfg.g == GG)                              \
+      return launch_x2_t<V, C, GG, LL>(g, v, cfg.ty, Tn, Ts, vmap, vtab, sfield, ry, s);
   HS2_X2(1, 16, 8) HS2_X2(2, 16, 8) HS2_X2(4, 16, 8) HS2_X2(8, 16, 8) HS2_X2(16, 16, 8)
   HS2_X2(4, 16, 16) HS2_X2(8, 16, 16) HS2_X2(16, 16, 4) HS2_X2(16, 16, 16)
   HS2_X2(8, 32, 4) HS2_X2(16, 32, 4) HS2_X2(16, 32, 8) HS2_X2(16, 32, 2) HS2_X2(16, 64, 2)
@@ -1081,11 +1066,13 @@ hipError_t launch_sweep_x(XConfig cfg, const Grid &g, const ClassView &v, const 
 hipError_t launch_sweep_x(XConfig cfg, const Grid &g, const DenseView &v, const double *Tn,
                           double *Ts, const uint8_t *vmap, const double *vtab,
                           const double *sfield, hipStream_t s, bool ry) {
+  if (dense_rows_ok(g)) return launch_dense_x(g, v, Tn, Ts, vmap, vtab, sfield, ry, s);
   return launch_x_v(cfg, g, v, Tn, Ts, vmap, vtab, sfield, ry, s);
 }
 hipError_t launch_sweep_x(XConfig cfg, const Grid &g, const AsymView &v, const double *Tn,
                           double *Ts, const uint8_t *vmap, const double *vtab,
                           const double *sfield, hipStream_t s, bool ry) {
+  if (dense_rows_ok(g)) return launch_dense_x(g, v, Tn, Ts, vmap, vtab, sfield, ry, s);
   return launch_x_v(cfg, g, v, Tn, Ts, vmap, vtab, sfield, ry, s);
 }
 
@@ -1147,10 +1134,14 @@ template <class V>
 static hipError_t launch_s_v(SConfig cfg, const Grid &g, const V &v, int axis, const double *Tn,
                              const double *Y, double *X, double *surf, double dz, bool ry,
                              hipStream_t s) {
+  // per-voxel columns come here beyond 512 cells, where P x CW <= 512 with CW
+  // >= 8 leaves segments of 16 and more
+  if constexpr (std::is_same<V, ClassView>::value) {
+    if (cfg.seg == 2) return launch_s_t<V, 2>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
+    if (cfg.seg == 4) return launch_s_t<V, 4>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
+    if (cfg.seg == 8) return launch_s_t<V, 8>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
+  }
   switch (cfg.seg) {
-    case 2: return launch_s_t<V, 2>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
-    case 4: return launch_s_t<V, 4>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
-    case 8: return launch_s_t<V, 8>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     case 16: return launch_s_t<V, 16>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     case 32: return launch_s_t<V, 32>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     default: return hipErrorInvalidValue;
@@ -1165,11 +1156,13 @@ hipError_t launch_sweep_strided(SConfig cfg, const Grid &g, const ClassView &v, 
 hipError_t launch_sweep_strided(SConfig cfg, const Grid &g, const DenseView &v, int axis,
                                 const double *Tn, const double *Y, double *X, double *surf,
                                 double dz, hipStream_t s, bool ry) {
+  if (dense_cols_ok(g, axis)) return launch_dense_cols(g, v, axis, Tn, Y, X, surf, dz, ry, s);
   return launch_s_v(cfg, g, v, axis, Tn, Y, X, surf, dz, ry, s);
 }
 hipError_t launch_sweep_strided(SConfig cfg, const Grid &g, const AsymView &v, int axis,
                                 const double *Tn, const double *Y, double *X, double *surf,
                                 double dz, hipStream_t s, bool ry) {
+  if (dense_cols_ok(g, axis)) return launch_dense_cols(g, v, axis, Tn, Y, X, surf, dz, ry, s);
   return launch_s_v(cfg, g, v, axis, Tn, Y, X, surf, dz, ry, s);
 }
 
@@ -1253,90 +1246,6 @@ hipError_t launch_surface(const double *T, int ny, int nx, double dz, double *ou
   int blocks = (sxy + 255) / 256;
   if (blocks > 65536) blocks = 65536;
   hipLaunchKernelGGL(k_surface, dim3(blocks), dim3(256), 0, s, T, ny, nx, dz, out);
-  return hipGetLastError();
-}
-
-
-// ------------------------------------------------------ batched sweeps
-// One launch covers every instance of a batch (per-voxel coefficients,
-// axis lengths <= kBatchMaxLen); see hs2_batch.h for the block mapping.
-// Lines of T^t of one x-sweep block (LPB whole x-lines, contiguous) copied
-// into the instance's checkpoint slot when step t starts a checkpoint
-// segment: (nsteps - t) % K == 0, or t == 0 (the segments are aligned to
-// the instance's end).
-__device__ __forceinline__ void batch_ckpt_lines(const BatchMap &m, const BatchInst &I, int t,
-                                                 int local, int lpb, const double *T,
-                                                 double *ck) {
-  const int r = I.nsteps - t;
-  if (r % m.K != 0 && t != 0) return;
-  const long long n = (long long)I.nz * I.ny * I.nx;
-  const int slot = (r + m.K - 1) / m.K - 1;
-  const long long c0 = (long long)local * lpb * I.nx;
-  const long long c1 = min(n, c0 + (long long)lpb * I.nx);
-  double *dst = ck + I.ckoff + (long long)slot * n;
-  for (long long c = c0 + threadIdx.x; c < c1; c += blockDim.x) dst[c] = T[I.off + c];
-}
-
-template <int G, int LPB>
-__global__ __launch_bounds__(G *LPB) void kb_sweep_x2(BatchMap m, DenseView v, const double *Tn,
-                                                     double *Ts, const double *src, double *ck) {
-  BatchInst I;
-  int local, t;
-  if (!batch_locate(m, I, local, t)) return;
-  if (ck) batch_ckpt_lines(m, I, t, local, LPB, Tn, ck);
-  const double *sf = (src && t == I.src_step) ? src + I.off : nullptr;
-  const Grid g{I.nz, I.ny, I.nx};
-  const DenseView vi = offset_view(v, I.off);
-  // lanes hold 2, 4 or 8 cells: 16 lanes cover the instance's x lines
-  switch (I.xseg) {
-    case 2:
-      sweep_x2_body<DenseView, 2, G, LPB, true>(g, vi, Tn + I.off, Ts + I.off, nullptr, nullptr,
-                                                sf, local, 0);
-      break;
-    case 4:
-      sweep_x2_body<DenseView, 4, G, LPB, true>(g, vi, Tn + I.off, Ts + I.off, nullptr, nullptr,
-                                                sf, local, 0);
-      break;
-    default:
-      sweep_x2_body<DenseView, 8, G, LPB, true>(g, vi, Tn + I.off, Ts + I.off, nullptr, nullptr,
-                                                sf, local, 0);
-      break;
-  }
-}
-
-template <int SEG, int AXIS>
-__global__ __launch_bounds__(kBatchThreads) void kb_sweep_strided(
-    BatchMap m, DenseView v, const double *Tn, const double *Y, double *X, double *hist) {
-  BatchInst I;
-  int local, t;
-  if (!batch_locate(m, I, local, t)) return;
-  double *surf = (AXIS == 0 && hist) ? hist + I.hoff + (long long)t * I.ny * I.nx : nullptr;
-  sweep_strided_body<DenseView, SEG, AXIS, false, false, true>(
-      Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off), I.cw[AXIS], Tn + I.off, Y + I.off,
-      X + I.off, surf, I.dz, local, batch_line_segs(AXIS == 1 ? I.ny : I.nz));
-}
-
-hipError_t launch_batch_x2(const BatchMap &m, int nblocks, const DenseView &v, const double *Tn,
-                           double *Ts, const double *src, double *ck, hipStream_t s) {
-  constexpr int G = 16, LPB = kBatchXLines, SEGMAX = kBatchMaxLen / 16;
-  constexpr int RS = G * SEGMAX + ((G * SEGMAX) >> 4) + 1;
-  // vtab, right-hand sides, parked x entries (M, g as doubles, w as bytes)
-  const size_t shm = sizeof(double) * (kMaxVtab + 3 * LPB * RS) + (size_t)LPB * RS;
-  hipLaunchKernelGGL((kb_sweep_x2<G, LPB>), dim3(nblocks), dim3(G * LPB), shm, s, m, v, Tn, Ts,
-                     src, ck);
-  return hipGetLastError();
-}
-
-hipError_t launch_batch_strided(const BatchMap &m, int nblocks, int axis, const DenseView &v,
-                                const double *Tn, const double *Y, double *X, double *hist,
-                                hipStream_t s) {
-  const size_t shm = sizeof(double) * 6 * (size_t)kBatchThreads;
-  if (axis == 1)
-    hipLaunchKernelGGL((kb_sweep_strided<kBatchSeg, 1>), dim3(nblocks), dim3(kBatchThreads), shm,
-                       s, m, v, Tn, Y, X, hist);
-  else
-    hipLaunchKernelGGL((kb_sweep_strided<kBatchSeg, 0>), dim3(nblocks), dim3(kBatchThreads), shm,
-                       s, m, v, Tn, Y, X, hist);
   return hipGetLastError();
 }
 

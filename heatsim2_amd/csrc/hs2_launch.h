@@ -50,6 +50,27 @@ hipError_t launch_sweep_strided(SConfig cfg, const Grid &g, const AsymView &v, i
                                 const double *Tn, const double *Y, double *X, double *surf,
                                 double dz, hipStream_t s, bool ry = false);
 
+// per-voxel coefficients in fixed shapes (hs2_dense.hip), where they serve the
+// grid: x rows of up to 256 cells, y and z columns of up to 512
+bool dense_rows_ok(const Grid &g);
+bool dense_cols_ok(const Grid &g, int axis);
+bool dense_ry(const Grid &g);  // x may hand y its right-hand side
+hipError_t launch_dense_x(const Grid &g, const DenseView &v, const double *Tn, double *Ts,
+                          const uint8_t *vmap, const double *vtab, const double *sfield, bool ry,
+                          hipStream_t s);
+hipError_t launch_dense_x(const Grid &g, const AsymView &v, const double *Tn, double *Ts,
+                          const uint8_t *vmap, const double *vtab, const double *sfield, bool ry,
+                          hipStream_t s);
+hipError_t launch_dense_cols(const Grid &g, const DenseView &v, int axis, const double *Tn,
+                             const double *Y, double *X, double *surf, double dz, bool ry,
+                             hipStream_t s);
+hipError_t launch_dense_cols(const Grid &g, const AsymView &v, int axis, const double *Tn,
+                             const double *Y, double *X, double *surf, double dz, bool ry,
+                             hipStream_t s);
+// U = A_axis^{-T} (scale_m ? M R : R) along every line of `axis`
+hipError_t launch_dense_adj(const Grid &g, const DenseView &v, int axis, const double *R,
+                            int scale_m, double *U, hipStream_t s);
+
 // K0 of the combined plane: mark the (z, y, x) class triples that occur in a
 // 2^24-bit map, then give each cell the rank of its triple among them
 hipError_t launch_comb_mark(int n, const uint8_t *cz, const uint8_t *cy, const uint8_t *cx,

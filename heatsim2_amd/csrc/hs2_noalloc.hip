@@ -88,10 +88,11 @@ extern "C" int hs2_step_noalloc(const hs2_grid_desc *grid, const double *d_M, co
   dv.g[2] = d_gx;
   const hs2::Grid g{G.nz, G.ny, G.nx};
   hipStream_t s = (hipStream_t)stream;
+  const bool ry = hs2::dense_ry(g);
   // the kernels and launch shapes of hs2_step on a plan that was given these
   // coefficients with hs2_plan_set_dense
-  hipError_t e = hs2::launch_sweep_x(xc, g, dv, d_Tin, ws, nullptr, nullptr, d_sfield, s);
-  if (e == hipSuccess) e = hs2::launch_sweep_strided(yc, g, dv, 1, d_Tin, ws, ws, nullptr, G.dz, s);
+  hipError_t e = hs2::launch_sweep_x(xc, g, dv, d_Tin, ws, nullptr, nullptr, d_sfield, s, ry);
+  if (e == hipSuccess) e = hs2::launch_sweep_strided(yc, g, dv, 1, d_Tin, ws, ws, nullptr, G.dz, s, ry);
   if (e == hipSuccess) e = hs2::launch_sweep_strided(zc, g, dv, 0, d_Tin, ws, d_Tout, d_surf, G.dz, s);
   if (e != hipSuccess)
     return hs2::fail(HS2_E_HIP, "hs2_step_noalloc: kernel launch: %s", hipGetErrorString(e));
