@@ -19,6 +19,20 @@ struct AdjFields {
   double *gsrc;
 };
 
+// Up to kAdjGroup adjoint steps whose sensitivities are added in one pass
+// (per-voxel coefficients), latest first.  Step s of the group has T^t at
+// T - s N, T^{t+1} at T + N - s N, T* and T** at Tx - s N and Ty - s N, and the
+// transposed solves u_z, u_y, u_x at u + 3 s N, + N and + 2 N; gsrc[s] takes w u_x
+// when non-null.
+constexpr int kAdjGroup = 4;
+struct AdjGroup {
+  const double *T, *Tx, *Ty, *u;
+  double *gM;
+  double *gg[3];
+  double *gsrc[kAdjGroup];
+  long long N;
+};
+
 struct AdjLineConfig {
   int seg, cw;  // seg 0: unsupported line length
 };
@@ -34,6 +48,14 @@ hipError_t launch_adj_stencil(const Grid &g, const ClassView &v, const AdjFields
                               hipStream_t s);
 hipError_t launch_adj_stencil(const Grid &g, const DenseView &v, const AdjFields &f,
                               hipStream_t s);
+// per-voxel coefficients, where dense_cols_ok(g, 0): lambda of the step before
+// from the solves of the step after (ux null: none) and the readout adjoint gh
+// (null: none), and its transposed z solve (solve false: lambda itself)
+hipError_t launch_dense_lambda(const Grid &g, const DenseView &v, const double *ux,
+                               const double *uy, const double *uz, const double *gh, bool solve,
+                               double *U, hipStream_t s);
+hipError_t launch_dense_sens(const Grid &g, const DenseView &v, const AdjGroup &f, int cnt,
+                             hipStream_t s);
 hipError_t launch_lam_from_readout(const Grid &g, const double *ghist, double *lam,
                                    hipStream_t s);
 hipError_t launch_fill(double *a, size_t n, double v, hipStream_t s);

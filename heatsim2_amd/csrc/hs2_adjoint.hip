@@ -23,6 +23,11 @@
 // diagonally dominant, so A_a^T is strictly column dominant and the same
 // segment elimination + PCR solves it without pivoting.
 //
+// The stencil as it stands here serves class maps (and per-voxel z lines of more
+// than 512 cells); on per-voxel coefficients dJ/dT^n is formed where the next
+// z solve needs it and the sensitivities of several steps are added at once
+// (hs2_dense.hip).
+//
 // No upstream counterpart: heatsim2 has no gradients.
 #include <hip/hip_runtime.h>
 
@@ -319,23 +324,6 @@ hipError_t launch_fill(double *a, size_t n, double v, hipStream_t s) {
 
 
 // ------------------------------------------------------ batched adjoint
-// f: base pointers of the concatenated fields; f.ghist: base of the
-// concatenated dJ/dhist; f.gsrc: base of the concatenated source gradients.
-__global__ __launch_bounds__(256) void kb_adj_stencil(BatchMap m, DenseView v, AdjFields f) {
-  BatchInst I;
-  int local, t;
-  if (!batch_locate(m, I, local, t)) return;
-  const long long o = I.off;
-  AdjFields g = f;
-  g.Tn += o; g.Tx += o; g.Ty += o; g.Tn1 += o;
-  g.ux += o; g.uy += o; g.uz += o;
-  g.lam_out += o; g.gM += o;
-  g.gg[0] += o; g.gg[1] += o; g.gg[2] += o;
-  g.ghist = (f.ghist && t >= 1) ? f.ghist + I.hoff + (long long)(t - 1) * I.ny * I.nx : nullptr;
-  g.gsrc = (f.gsrc && t == I.src_step) ? f.gsrc + o : nullptr;
-  adj_stencil_body<DenseView>(Grid{I.nz, I.ny, I.nx}, offset_view(v, o), g, local);
-}
-
 // backward segment start: checkpoint of the segment -> segment slot K - (e - s)
 __global__ void kb_ckpt_load(BatchMap m, const double *ck, double *seg, long long N) {
   BatchInst I;
@@ -350,39 +338,14 @@ __global__ void kb_ckpt_load(BatchMap m, const double *ck, double *seg, long lon
   seg[(long long)slot * N + I.off + c] = ck[c];
 }
 
-// lam = readout adjoint of the last history row of each instance
-__global__ void kb_lam_init(BatchMap m, const double *ghist, double *lam) {
-  BatchInst I;
-  int local, t;
-  if (!batch_locate(m, I, local, t)) return;
-  const long long nyx = (long long)I.ny * I.nx, n = nyx * I.nz;
-  const long long c = (long long)local * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  const long long k = c / nyx, rem = c - k * nyx;
-  const double *gh = ghist + I.hoff + (long long)(I.nsteps - 1) * nyx;
-  lam[I.off + c] = k == 0 ? (21.0 / 16.0) * gh[rem] : k == 1 ? -(5.0 / 16.0) * gh[rem] : 0.0;
-}
-
 // ctr[which] = value (set) or += value (add); one thread
 __global__ void kb_counter(int *ctr, int which, int value, int add) {
   if (threadIdx.x == 0 && blockIdx.x == 0) ctr[which] = add ? ctr[which] + value : value;
 }
 
-hipError_t launch_batch_adj_stencil(const BatchMap &m, int nblocks, const DenseView &v,
-                                    const AdjFields &f, hipStream_t s) {
-  hipLaunchKernelGGL(kb_adj_stencil, dim3(nblocks), dim3(256), 0, s, m, v, f);
-  return hipGetLastError();
-}
-
 hipError_t launch_batch_ckpt_load(const BatchMap &m, int nblocks, const double *ck, double *seg,
                                   long long N, hipStream_t s) {
   hipLaunchKernelGGL(kb_ckpt_load, dim3(nblocks), dim3(256), 0, s, m, ck, seg, N);
-  return hipGetLastError();
-}
-
-hipError_t launch_batch_lam_init(const BatchMap &m, int nblocks, const double *ghist, double *lam,
-                                 hipStream_t s) {
-  hipLaunchKernelGGL(kb_lam_init, dim3(nblocks), dim3(256), 0, s, m, ghist, lam);
   return hipGetLastError();
 }
 

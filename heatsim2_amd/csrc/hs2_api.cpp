@@ -82,7 +82,7 @@ struct hs2_plan {
   hs2::SConfig scfg[2] = {{0, 0}, {0, 0}};  // [0] z, [1] y
 };
 
-enum { KIND_X2 = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, NKIND = 5 };
+enum { KIND_X2 = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, KIND_SENS = 5, NKIND = 6 };
 
 struct hs2_batch {
   int ninst = 0, K = 0, maxsteps = 0, device = 0;
@@ -270,6 +270,12 @@ hipError_t adj_stencil(const hs2_plan *p, const hs2::AdjFields &f, hipStream_t s
                                : hs2::launch_adj_stencil(grid_of(p), p->dv, f, s);
 }
 
+// the adjoint in groups of steps (lambda folded into the z solve, the
+// sensitivities of kAdjGroup steps in one pass)
+bool grad_grouped(const hs2_plan *p) {
+  return p->mode == MODE_DENSE && hs2::dense_cols_ok(grid_of(p), 0);
+}
+
 // step -> source index (-1: none); validates the schedule
 int source_schedule(int nsteps, const int32_t *h_src_step, int nsrc, const double *d_src,
                     std::vector<int> *out, const char *who) {
@@ -328,6 +334,9 @@ int blocks_of(const hs2::BatchInst &I, int kind) {
     case KIND_Y: return (I.nx * I.nz + I.cw[1] - 1) / I.cw[1];
     case KIND_Z: return (I.nx * I.ny + I.cw[0] - 1) / I.cw[0];
     case KIND_AX: return (I.rows + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
+    case KIND_SENS:
+      return (I.nx * I.ny + 255) / 256 *
+             ((I.nz + hs2::kBatchSensPlanes - 1) / hs2::kBatchSensPlanes);
     default: return (int)(((long long)I.nz * I.ny * I.nx + 255) / 256);
   }
 }
@@ -347,11 +356,13 @@ void batch_free(hs2_batch *b) {
 }
 
 // work layout: ws (N) | checkpoints (CK) | segment T^t (K+1 N) | T* (K N) | T** (K N) |
-// ux uy uz lam (4 N)
+// u_z u_y u_x of each step of a group (3 N each)
 struct BatchWork {
-  double *ws, *ck, *seg, *segx, *segy, *ux, *uy, *uz, *lam;
+  double *ws, *ck, *seg, *segx, *segy, *u;
 };
-long long batch_work_doubles(const hs2_batch *b) { return b->N * (3LL * b->K + 6) + b->CK; }
+long long batch_work_doubles(const hs2_batch *b) {
+  return b->N * (3LL * b->K + 2 + 3 * hs2::kAdjGroup) + b->CK;
+}
 BatchWork batch_work(const hs2_batch *b, double *w) {
   BatchWork r;
   r.ws = w;
@@ -359,10 +370,7 @@ BatchWork batch_work(const hs2_batch *b, double *w) {
   r.seg = r.ck + b->CK;
   r.segx = r.seg + (size_t)(b->K + 1) * b->N;
   r.segy = r.segx + (size_t)b->K * b->N;
-  r.ux = r.segy + (size_t)b->K * b->N;
-  r.uy = r.ux + b->N;
-  r.uz = r.uy + b->N;
-  r.lam = r.uz + b->N;
+  r.u = r.segy + (size_t)b->K * b->N;
   return r;
 }
 
@@ -405,30 +413,33 @@ hipError_t emit_backward_segment(hs2_batch *b, const double *src, const double *
       e = hs2::launch_batch_cols(batch_map(b, KIND_Z, hs2::RULE_RECOMP, j), b->nblk[KIND_Z], 0,
                                  b->dv, in, ty, w.seg + (size_t)(j + 1) * N, nullptr, false, s);
   }
-  // adjoint steps, latest first: z, y, x transposed line solves from
-  // lam = dJ/dT^{t+1}, then the stencil, which leaves dJ/dT^t in lam
+  // adjoint steps, latest first: lambda from the solves of the step after (the
+  // last one of the segment before has slot (K - 1) % S) and the z, y, x
+  // transposed solves; the sensitivities group by group
+  constexpr int S = hs2::kAdjGroup;
   for (int j = 0; j < K && e == hipSuccess; j++) {
-    const size_t q = (size_t)(K - 1 - j);
-    e = hs2::launch_batch_adj_line(batch_map(b, KIND_Z, hs2::RULE_BWD, j), b->nblk[KIND_Z], 0,
-                                   b->dv, w.lam, 0, w.uz, s);
+    double *uz = w.u + (size_t)(j % S) * 3 * N, *uy = uz + N, *ux = uy + N;
+    const double *after = w.u + (size_t)((j > 0 ? j - 1 : K - 1) % S) * 3 * N;
+    e = hs2::launch_batch_lambda(batch_map(b, KIND_Z, hs2::RULE_BWD, j), b->nblk[KIND_Z], b->dv,
+                                 after, b->N, ghist, uz, s);
     if (e == hipSuccess)
       e = hs2::launch_batch_adj_line(batch_map(b, KIND_Y, hs2::RULE_BWD, j), b->nblk[KIND_Y], 1,
-                                     b->dv, w.uz, 1, w.uy, s);
+                                     b->dv, uz, 1, uy, s);
     if (e == hipSuccess)
       e = hs2::launch_batch_adj_line(batch_map(b, KIND_AX, hs2::RULE_BWD, j), b->nblk[KIND_AX], 2,
-                                     b->dv, w.uy, 1, w.ux, s);
-    if (e == hipSuccess) {
-      hs2::AdjFields f{};
-      f.Tn = w.seg + q * N; f.Tx = w.segx + q * N; f.Ty = w.segy + q * N;
-      f.Tn1 = w.seg + (q + 1) * N;
-      f.ux = w.ux; f.uy = w.uy; f.uz = w.uz;
-      f.ghist = ghist;
-      f.lam_out = w.lam;
+                                     b->dv, uy, 1, ux, s);
+    if (e == hipSuccess && (j % S == S - 1 || j == K - 1)) {
+      const int j0 = j - j % S;
+      const size_t q = (size_t)(K - 1 - j0);
+      hs2::AdjGroup f{};
+      f.T = w.seg + q * N; f.Tx = w.segx + q * N; f.Ty = w.segy + q * N;
+      f.u = w.u;
       f.gM = gM;
       f.gg[0] = gz; f.gg[1] = gy; f.gg[2] = gx;
-      f.gsrc = gsrc;
-      e = hs2::launch_batch_adj_stencil(batch_map(b, KIND_CELL, hs2::RULE_BWD, j),
-                                        b->nblk[KIND_CELL], b->dv, f, s);
+      for (double *&gs : f.gsrc) gs = gsrc;
+      f.N = b->N;
+      e = hs2::launch_batch_sens(batch_map(b, KIND_SENS, hs2::RULE_BWD, j0), b->nblk[KIND_SENS],
+                                 b->dv, f, j - j0 + 1, s);
     }
   }
   if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 1, 1, 1, s);
@@ -1211,7 +1222,7 @@ int hs2_run_timed(hs2_plan *p, double *d_T, int nsteps, int method, double *kern
 
 size_t hs2_grad_work_doubles(const hs2_plan *p, int ckpt_every) {
   if (!p || ckpt_every < 1) return 0;
-  return (3 * (size_t)ckpt_every + 6) * (size_t)p->n;
+  return (3 * (size_t)ckpt_every + (grad_grouped(p) ? 1 + 3 * hs2::kAdjGroup : 6)) * (size_t)p->n;
 }
 
 int hs2_grad_forward(hs2_plan *p, double *d_T, int nsteps, int ckpt_every, double *d_ckpt,
@@ -1255,7 +1266,7 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
   if (p->grid.nz < 2) return fail(HS2_E_ARG, "hs2_grad_backward: the surface readout needs nz >= 2");
   if (!aligned16(d_ckpt) || !aligned16(d_work))
     return fail(HS2_E_ARG, "hs2_grad_backward: d_ckpt and d_work must be 16-byte aligned");
-  const size_t need = hs2_grad_work_doubles(p, ckpt_every);
+  const size_t need = (3 * (size_t)ckpt_every + 6) * (size_t)p->n;
   if (work_doubles < need)
     return fail(HS2_E_ARG, "hs2_grad_backward: work buffer has %zu doubles, needs %zu",
                 work_doubles, need);
@@ -1273,13 +1284,20 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
   // its K steps, so every state of the segment is computed once
   double *seg = d_work;
   double *segx = seg + (size_t)(K + 1) * n, *segy = segx + (size_t)K * n;
-  double *ux = segy + (size_t)K * n, *uy = ux + n, *uz = uy + n;
-  double *lam = uz + n, *lam2 = lam + n;
+  // per-voxel coefficients: the solves of a group of steps; class maps: u_x,
+  // u_y, u_z of one step, lambda and the next lambda
+  double *u = segy + (size_t)K * n;
+  double *ux = u, *uy = ux + n, *uz = uy + n, *lam = uz + n, *lam2 = lam + n;
+  const bool grouped = grad_grouped(p);
+  // steps of a group: as many as the workspace has room for (at least one)
+  const int S = (int)std::min<size_t>(hs2::kAdjGroup, (work_doubles / n - (3 * (size_t)K + 1)) / 3);
+  const double *after = nullptr;  // grouped: the solves of the step after
   HIP_TRY(hs2::launch_fill(d_gM, n, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gz, n, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gy, n, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gx, n, 0.0, s));
-  HIP_TRY(hs2::launch_lam_from_readout(g, d_grad_hist + (size_t)(nsteps - 1) * nyx, lam, s));
+  if (!grouped)
+    HIP_TRY(hs2::launch_lam_from_readout(g, d_grad_hist + (size_t)(nsteps - 1) * nyx, lam, s));
   const int nseg = (nsteps + K - 1) / K;
   for (int sg = nseg - 1; sg >= 0; sg--) {
     const int n0 = sg * K, n1 = std::min(nsteps, n0 + K);
@@ -1292,7 +1310,29 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
                        nullptr, s);
       if (rc != HS2_OK) return rc;
     }
-    for (int t = n1 - 1; t >= n0; t--) {
+    for (int t = n1 - 1; grouped && t >= n0; t--) {
+      const int slot = (n1 - 1 - t) % S;
+      double *wz = u + (size_t)slot * 3 * n, *wy = wz + n, *wx = wy + n;
+      HIP_TRY(hs2::launch_dense_lambda(g, p->dv, after ? after + 2 * n : nullptr,
+                                       after ? after + n : nullptr, after, d_grad_hist + (size_t)t * nyx, true, wz, s));
+      HIP_TRY(adj_line(p, 1, wz, 1, wy, s));
+      HIP_TRY(adj_line(p, 2, wy, 1, wx, s));
+      after = wz;
+      if (slot < S - 1 && t > n0) continue;
+      const size_t q = (size_t)(t + slot - n0);  // the group's latest step
+      hs2::AdjGroup f{};
+      f.T = seg + q * n; f.Tx = segx + q * n; f.Ty = segy + q * n;
+      f.u = u;
+      f.gM = d_gM;
+      f.gg[0] = d_gz; f.gg[1] = d_gy; f.gg[2] = d_gx;
+      for (int i = 0; i <= slot; i++) {
+        const int at = src[t + slot - i];
+        f.gsrc[i] = at >= 0 ? d_gsrc + (size_t)at * n : nullptr;
+      }
+      f.N = (long long)n;
+      HIP_TRY(hs2::launch_dense_sens(g, p->dv, f, slot + 1, s));
+    }
+    for (int t = n1 - 1; !grouped && t >= n0; t--) {
       const size_t q = (size_t)(t - n0);
       HIP_TRY(adj_line(p, 0, lam, 0, uz, s));
       HIP_TRY(adj_line(p, 1, uz, 1, uy, s));
@@ -1309,7 +1349,10 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
       std::swap(lam, lam2);
     }
   }
-  if (d_gT0)
+  if (d_gT0 && grouped)
+    HIP_TRY(hs2::launch_dense_lambda(g, p->dv, after + 2 * n, after + n, after, nullptr, false,
+                                     d_gT0, s));
+  else if (d_gT0)
     HIP_TRY(hipMemcpyAsync(d_gT0, lam, n * sizeof(double), hipMemcpyDeviceToDevice, s));
   return HS2_OK;
 }
@@ -1485,8 +1528,6 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   HIP_TRY(hs2::launch_fill(d_gy, b->N, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gx, b->N, 0.0, s));
   if (d_gsrc) HIP_TRY(hs2::launch_fill(d_gsrc, b->N, 0.0, s));
-  HIP_TRY(hs2::launch_batch_lam_init(batch_map(b, KIND_CELL, hs2::RULE_ALL, 0), b->nblk[KIND_CELL],
-                                     d_grad_hist, w.lam, s));
   HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 1, 0, 0, s));
   const int reps = (b->maxsteps + b->K - 1) / b->K;
   const std::vector<const void *> key = {d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc,

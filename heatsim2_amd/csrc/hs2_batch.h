@@ -24,6 +24,7 @@ constexpr int kBatchThreads = 256; // threads per block of the y and z kernels
 constexpr int kBatchWaves = 4;     // waves (units of rows) per block of the x kernels
 constexpr int kBatchSeg = 8;       // cells per thread segment of the line kernels
 constexpr int kBatchPlanes = 2;    // planes a wave of the x sweep walks (1, 4: 2% slower, 8: 18%)
+constexpr int kBatchSensPlanes = 8;  // planes per block of the sensitivity pass
 constexpr int kBatchAlign = 32;    // instance offsets are multiples of this many cells
 
 // Segments of kBatchSeg cells per line of L cells in the y and z line
@@ -116,7 +117,7 @@ __device__ __forceinline__ DenseView offset_view(DenseView v, long long off) {
 }  // namespace hs2
 
 namespace hs2 {
-struct AdjFields;
+struct AdjGroup;
 // launchers (hs2_kernels.hip, hs2_adjoint.hip); nblocks = this kind's block total
 // the x sweep; with ck != nullptr (forward) T^t is copied into the instance's
 // checkpoint slot on a checkpoint step; ry as for a plan's sweeps
@@ -127,11 +128,11 @@ hipError_t launch_batch_cols(const BatchMap &m, int nblocks, int axis, const Den
                              hipStream_t s);
 hipError_t launch_batch_adj_line(const BatchMap &m, int nblocks, int axis, const DenseView &v,
                                  const double *R, int scale_m, double *U, hipStream_t s);
-hipError_t launch_batch_adj_stencil(const BatchMap &m, int nblocks, const DenseView &v,
-                                    const AdjFields &f, hipStream_t s);
+hipError_t launch_batch_lambda(const BatchMap &m, int nblocks, const DenseView &v, const double *u,
+                               long long N, const double *ghist, double *U, hipStream_t s);
+hipError_t launch_batch_sens(const BatchMap &m, int nblocks, const DenseView &v, const AdjGroup &f,
+                             int cnt, hipStream_t s);
 hipError_t launch_batch_ckpt_load(const BatchMap &m, int nblocks, const double *ck, double *seg,
                                   long long N, hipStream_t s);
-hipError_t launch_batch_lam_init(const BatchMap &m, int nblocks, const double *ghist, double *lam,
-                                 hipStream_t s);
 hipError_t launch_batch_counter(int *ctr, int which, int value, int add, hipStream_t s);
 }  // namespace hs2

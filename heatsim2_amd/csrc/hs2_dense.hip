@@ -315,6 +315,196 @@ __device__ __forceinline__ void col_adjoint(const Grid &g, const V &v, int P, in
   }
 }
 
+// dJ/dT^{t+1} (lambda) of the cells of a block's z columns, and its transposed
+// z solve: A_z^T U = lambda.  lambda is the adjoint stencil of the step after
+// (its transposed solves ux, uy, uz; null: no such step) plus the readout
+// adjoint `gh` of T^{t+1} on the top two layers.  U may be uz: a block reads uz
+// in its own columns only, before its first barrier.  SOLVE false: lambda is
+// the result.
+//
+// One pass instead of the adjoint stencil's lambda and the z solve that read it
+// back (65 bytes a cell; those moved 98).  Memory and latency bound at three
+// waves a SIMD: all of a segment's loads are issued together (about 160
+// registers).  Fewer registers lose: 128 by spilling 24.2 us, 150 by loading
+// the y faces after the x faces are done 18.3, as it stands 15.3 (64x128x128).
+template <int SEG, bool SOLVE>
+__device__ __forceinline__ void col_lambda(const Grid &g, const DenseView &v, int P, int CW,
+                                           const double *ux, const double *uy, const double *uz,
+                                           const double *gh, double *U, int blk) {
+  extern __shared__ double lds[];
+  const ColPlace c = col_place<0>(g, SEG, P, CW, blk);
+  const int nx = g.nx, j = c.base / nx, i = c.base - j * nx;
+  const unsigned n = (unsigned)nx * (unsigned)g.ny * (unsigned)g.nz;
+  const BufRsrc bU = make_buf(U, n * 8u), bM = make_buf(v.M, n * 8u),
+                bGz = make_buf(v.g[0], n * 8u), bW = make_buf(v.w, n);
+  const unsigned so = c.so * 8u, vo = c.vo * 8u, row = (unsigned)nx;
+  double M[SEG], G[SEG + 1], lam[SEG];
+  uint32_t w[SEG + 2];
+#pragma unroll
+  for (int q = 0; q < SEG; q++) M[q] = buf_load_d(bM, vo + q * so);
+#pragma unroll
+  for (int q = 0; q <= SEG; q++) G[q] = buf_load_d(bGz, vo + q * so);
+  w[0] = buf_load_u8(bW, c.t0 > 0 ? c.vo - c.so : c.vo);
+#pragma unroll
+  for (int q = 0; q <= SEG; q++) w[q + 1] = buf_load_u8(bW, c.vo + q * c.so);
+  if (ux) {
+    // v across the faces of each axis: x: w ux / 2, y: w (ux - uy / 2), z:
+    // w (ux - uz / 2); faces that are not there add nothing (an offset before
+    // the array or behind it reads 0)
+    const BufRsrc bX = make_buf(ux, n * 8u), bY = make_buf(uy, n * 8u), bZ = make_buf(uz, n * 8u),
+                  bGx = make_buf(v.g[2], n * 8u), bGy = make_buf(v.g[1], n * 8u);
+    double x[SEG], vz[SEG + 2];
+    {
+      const unsigned om = c.t0 > 0 ? vo - so : vo;
+      vz[0] = (double)w[0] * (buf_load_d(bX, om) - 0.5 * buf_load_d(bZ, om));
+    }
+#pragma unroll
+    for (int q = 0; q <= SEG; q++) {
+      const double xq = buf_load_d(bX, vo + q * so);
+      if (q < SEG) x[q] = xq;
+      vz[q + 1] = (double)w[q + 1] * (xq - 0.5 * buf_load_d(bZ, vo + q * so));
+    }
+#pragma unroll
+    for (int q = 0; q < SEG; q++) {
+      const int t = c.t0 + q;
+      const double dm = t > 0 ? vz[q] - vz[q + 1] : 0.0;
+      const double dp = t + 1 < c.L ? vz[q + 2] - vz[q + 1] : 0.0;
+      lam[q] = __builtin_fma(G[q + 1], dp, __builtin_fma(G[q], dm, M[q] * x[q]));
+    }
+#pragma unroll
+    for (int q = 0; q < SEG; q++) {
+      const unsigned o = vo + q * so, ow = c.vo + q * c.so;
+      const double vc = 0.5 * (double)w[q + 1] * x[q];
+      const double vm = 0.5 * (double)buf_load_u8(bW, ow - 1u) * buf_load_d(bX, o - 8u);
+      const double vp = 0.5 * (double)buf_load_u8(bW, ow + 1u) * buf_load_d(bX, o + 8u);
+      const double dm = i > 0 ? vm - vc : 0.0, dp = i + 1 < nx ? vp - vc : 0.0;
+      lam[q] = __builtin_fma(buf_load_d(bGx, o + 8u), dp,
+                             __builtin_fma(buf_load_d(bGx, o), dm, lam[q]));
+    }
+#pragma unroll
+    for (int q = 0; q < SEG; q++) {
+      const unsigned o = vo + q * so, ow = c.vo + q * c.so;
+      const double vc = (double)w[q + 1] * (x[q] - 0.5 * buf_load_d(bY, o));
+      const double vm = (double)buf_load_u8(bW, ow - row) *
+                        (buf_load_d(bX, o - 8u * row) - 0.5 * buf_load_d(bY, o - 8u * row));
+      const double vp = (double)buf_load_u8(bW, ow + row) *
+                        (buf_load_d(bX, o + 8u * row) - 0.5 * buf_load_d(bY, o + 8u * row));
+      const double dm = j > 0 ? vm - vc : 0.0, dp = j + 1 < g.ny ? vp - vc : 0.0;
+      lam[q] = __builtin_fma(buf_load_d(bGy, o + 8u * row), dp,
+                             __builtin_fma(buf_load_d(bGy, o), dm, lam[q]));
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < SEG; q++) lam[q] = 0.0;
+  }
+  if (gh && c.t0 == 0) {
+    const double s = gh[c.base];
+    lam[0] = __builtin_fma(21.0 / 16.0, s, lam[0]);
+    lam[1] = __builtin_fma(-5.0 / 16.0, s, lam[1]);
+  }
+  if constexpr (!SOLVE) {
+    if (!c.valid) return;
+#pragma unroll
+    for (int q = 0; q < SEG; q++)
+      if (c.t0 + q < c.L) buf_store_ds(lam[q], bU, vo, q * so);
+  } else {
+    Seg<SEG> seg;
+#pragma unroll
+    for (int q = 0; q < SEG; q++) {
+      const int t = c.t0 + q;
+      const bool in = t < c.L;
+      const double gm = t > 0 ? G[q] : 0.0;
+      const double gp = t + 1 < c.L ? G[q + 1] : 0.0;
+      const double b = M[q] + 0.5 * (double)w[q + 1] * (gm + gp);
+      seg.row(q, in ? -0.5 * (double)w[q] * gm : 0.0, in ? b : 1.0,
+              in ? -0.5 * (double)w[q + 2] * gp : 0.0, in ? lam[q] : 0.0);
+    }
+    double As, Cs, Rs, Ae, Ce, Re, xs = 0.0, xe = 0.0;
+    seg.finish(As, Cs, Rs, Ae, Ce, Re);
+    block_ends(lds, c.p, P, CW, c.cl, c.act, As, Cs, Rs, Ae, Ce, Re, xs, xe);
+    if (!c.valid) return;
+#pragma unroll
+    for (int q = 0; q < SEG; q++) {
+      const double y = q == 0 ? xs : q == SEG - 1 ? xe : seg.interior(q, xs, xe);
+      if (c.t0 + q < c.L) buf_store_ds(y, bU, vo, q * so);
+    }
+  }
+}
+
+// Sensitivities of up to kAdjGroup adjoint steps added to the four gradient
+// fields, latest step first: one pass over the fields for the group instead of
+// one for every step.  A thread owns one column of planes k0 .. k1 - 1 and
+// carries the plane before in registers.
+//
+// Bound by memory: (25 fields read, 4 of them read and written, and w for four
+// steps) 265 bytes a cell in 52 us at 64x128x128, 5.3 TB/s.  lambda, the z
+// solve and this take 28 us a step there, where a stencil that added every
+// step by itself took 35.3 and the z solve 7.9; a batch of 24 instances of
+// 32..128^3 went from 298 to 243.  Groups of eight read 13% less a step but
+// run slower at 64x128x128 (102 us) and gain 1% of the whole in the batch,
+// for 12 more fields of workspace.
+__device__ __forceinline__ void add_sensitivities(const Grid &g, const uint8_t *__restrict__ w,
+                                                  const AdjGroup &f, int cnt, int col, int k0,
+                                                  int k1) {
+  constexpr int S = kAdjGroup;
+  const int nx = g.nx, sxy = nx * g.ny;
+  if (col >= sxy) return;
+  const int j = col / nx, i = col - j * nx;
+  const double *__restrict__ T = f.T, *__restrict__ Tx = f.Tx, *__restrict__ Ty = f.Ty,
+               *__restrict__ u = f.u;
+  const long long N = f.N;
+  // of the plane before: T^{t+1} of the latest step and every T^t, w ux, w uz
+  double bT[S + 1] = {}, bX[S] = {}, bZ[S] = {};
+  if (k0 > 0) {
+    const int c = (k0 - 1) * sxy + col;
+    const double wc = w[c];
+    bT[0] = T[N + c];
+#pragma unroll
+    for (int s = 0; s < S; s++)
+      if (s < cnt) {
+        bT[s + 1] = T[c - s * N];
+        bZ[s] = wc * u[3 * s * N + c];
+        bX[s] = wc * u[(3 * s + 2) * N + c];
+      }
+  }
+  for (int k = k0; k < k1; k++) {
+    const int c = k * sxy + col, cx = i > 0 ? c - 1 : c, cy = j > 0 ? c - nx : c;
+    const double wc = w[c], wx = w[cx], wy = w[cy];
+    double aM = f.gM[c], az = f.gg[0][c], ay = f.gg[1][c], ax = f.gg[2][c];
+    double T1 = T[N + c], T1b = bT[0];
+    bT[0] = T1;
+#pragma unroll
+    for (int s = 0; s < S; s++)
+      if (s < cnt) {
+        const double *Ts = T - s * N, *Xs = Tx - s * N, *Ys = Ty - s * N;
+        const double *uz = u + 3 * s * N, *uy = uz + N, *ux = uy + N;
+        const double Tn = Ts[c], X = Xs[c], Y = Ys[c], z = uz[c], y = uy[c], x = ux[c];
+        const double wz_ = wc * z, wy_ = wc * y, wx_ = wc * x;
+        aM -= x * (X - Tn) + y * (Y - X) + z * (T1 - Y);
+        const double gx = 0.5 * ((X + Tn) - (Xs[cx] + Ts[cx])) * (wx * ux[cx] - wx_);
+        ax += i > 0 ? gx : 0.0;
+        const double Tm = Ts[cy];
+        const double gy = (Tn - Tm) * (wy * ux[cy] - wx_) +
+                          0.5 * ((Y - Tn) - (Ys[cy] - Tm)) * (wy * uy[cy] - wy_);
+        ay += j > 0 ? gy : 0.0;
+        const double Tb = bT[s + 1];
+        const double gz =
+            (Tn - Tb) * (bX[s] - wx_) + 0.5 * ((T1 - Tn) - (T1b - Tb)) * (bZ[s] - wz_);
+        az += k > 0 ? gz : 0.0;
+        if (f.gsrc[s]) f.gsrc[s][c] = wx_;
+        T1 = Tn;
+        T1b = Tb;
+        bT[s + 1] = Tn;
+        bX[s] = wx_;
+        bZ[s] = wz_;
+      }
+    f.gM[c] = aM;
+    f.gg[0][c] = az;
+    f.gg[1][c] = ay;
+    f.gg[2][c] = ax;
+  }
+}
+
 // -------------------------------------------------------- single plans
 template <class V, int CPL, int G, bool SRC, bool RY>
 __global__ __launch_bounds__(256) void k_drows(Grid g, V v, const double *Tn, double *Ts,
@@ -352,6 +542,21 @@ __global__ __launch_bounds__(512) void k_dcols_adj(Grid g, V v, int P, int CW, c
                                                    int scale_m, double *U) {
   col_adjoint<V, SEG, AXIS>(g, v, P, CW, R, scale_m, U,
                             xcd_remap_chunks<32>(blockIdx.x, gridDim.x));
+}
+
+template <int SEG, bool SOLVE>
+__global__ __launch_bounds__(512) void k_dlambda(Grid g, DenseView v, int P, int CW,
+                                                 const double *ux, const double *uy,
+                                                 const double *uz, const double *gh, double *U) {
+  col_lambda<SEG, SOLVE>(g, v, P, CW, ux, uy, uz, gh, U,
+                         xcd_remap_chunks<32>(blockIdx.x, gridDim.x));
+}
+
+__global__ __launch_bounds__(256) void k_dsens(Grid g, const uint8_t *w, AdjGroup f, int cnt,
+                                               int KZ, int nbp) {
+  const int b = xcd_remap_chunks<32>(blockIdx.x, gridDim.x), kc = b / nbp;
+  add_sensitivities(g, w, f, cnt, (b - kc * nbp) * 256 + (int)threadIdx.x, kc * KZ,
+                    min(kc * KZ + KZ, g.nz));
 }
 
 // cells per lane and lanes of a row of nx cells (0: none).  Twice the lanes at
@@ -505,6 +710,32 @@ hipError_t launch_dense_adj(const Grid &g, const DenseView &v, int axis, const d
   return hipGetLastError();
 }
 
+hipError_t launch_dense_lambda(const Grid &g, const DenseView &v, const double *ux,
+                               const double *uy, const double *uz, const double *gh, bool solve,
+                               double *U, hipStream_t s) {
+  int seg, P, CW;
+  const long long ncol = (long long)g.nx * g.ny;
+  dcol_shape(g.nz, ncol, &seg, &P, &CW);
+  const dim3 grid((unsigned)((ncol + CW - 1) / CW)), block(P * CW);
+  const size_t shm = sizeof(double) * 6 * P * CW;
+#define HS2_RUN(SEG, SOLVE)                                                                   \
+  if (seg == SEG && solve == SOLVE)                                                           \
+    hipLaunchKernelGGL((k_dlambda<SEG, SOLVE>), grid, block, shm, s, g, v, P, CW, ux, uy, uz, gh, \
+                       U);
+  HS2_RUN(8, true) HS2_RUN(8, false) HS2_RUN(16, true) HS2_RUN(16, false)
+#undef HS2_RUN
+  return hipGetLastError();
+}
+
+hipError_t launch_dense_sens(const Grid &g, const DenseView &v, const AdjGroup &f, int cnt,
+                             hipStream_t s) {
+  const int nbp = (g.nx * g.ny + 255) / 256;
+  const int KZ = std::clamp(nbp * 4 * g.nz / 2048, 1, 16);
+  hipLaunchKernelGGL(k_dsens, dim3((unsigned)(nbp * ((g.nz + KZ - 1) / KZ))), dim3(256), 0, s, g,
+                     v.w, f, cnt, KZ, nbp);
+  return hipGetLastError();
+}
+
 // -------------------------------------------------------------- batches
 // One launch covers every instance (axis lengths <= kBatchMaxLen); see
 // hs2_batch.h for the block mapping.
@@ -578,6 +809,53 @@ __global__ __launch_bounds__(kBatchThreads) void kb_cols_adj(BatchMap m, DenseVi
   col_adjoint<DenseView, kBatchSeg, AXIS>(
       Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off), batch_line_segs(AXIS == 1 ? I.ny : I.nz),
       I.cw[AXIS], R + I.off, scale_m, U + I.off, local);
+}
+
+// u: the previous step's solves (uz, uy, ux, N apart); in the last step of an
+// instance (segment 0, j = 0) lambda is the readout adjoint alone.
+__global__ __launch_bounds__(kBatchThreads) void kb_lambda(BatchMap m, DenseView v,
+                                                           const double *u, long long N,
+                                                           const double *ghist, double *U) {
+  BatchInst I;
+  int local, t;
+  if (!batch_locate(m, I, local, t)) return;
+  const double *uz = u + I.off;
+  const bool last = t + 1 == I.nsteps;
+  col_lambda<kBatchSeg, true>(Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off),
+                              batch_line_segs(I.nz), I.cw[0], last ? nullptr : uz + 2 * N,
+                              uz + N, uz, ghist + I.hoff + (long long)t * I.ny * I.nx,
+                              U + I.off, local);
+}
+
+// f: base pointers of the concatenated fields; the group's steps are j = m.j to
+// m.j + cnt - 1 of the segment
+__global__ __launch_bounds__(256) void kb_sens(BatchMap m, const uint8_t *w, AdjGroup f, int cnt) {
+  BatchInst I;
+  int local, t;
+  if (!batch_locate(m, I, local, t)) return;
+  const int first = max(0, I.nsteps - (m.ctr[1] + 1) * m.K);  // the segment's first step
+  const long long o = I.off;
+  f.T += o; f.Tx += o; f.Ty += o; f.u += o;
+  f.gM += o; f.gg[0] += o; f.gg[1] += o; f.gg[2] += o;
+#pragma unroll
+  for (int s = 0; s < kAdjGroup; s++)
+    f.gsrc[s] = f.gsrc[s] && t - s == I.src_step ? f.gsrc[s] + o : nullptr;
+  const int nbp = (I.nx * I.ny + 255) / 256, kc = local / nbp;
+  add_sensitivities(Grid{I.nz, I.ny, I.nx}, w + o, f, min(cnt, t - first + 1),
+                    (local - kc * nbp) * 256 + (int)threadIdx.x, kc * kBatchSensPlanes,
+                    min((kc + 1) * kBatchSensPlanes, I.nz));
+}
+
+hipError_t launch_batch_lambda(const BatchMap &m, int nblocks, const DenseView &v, const double *u,
+                               long long N, const double *ghist, double *U, hipStream_t s) {
+  hipLaunchKernelGGL(kb_lambda, dim3(nblocks), dim3(kBatchThreads),
+                     sizeof(double) * 6 * (size_t)kBatchThreads, s, m, v, u, N, ghist, U);
+  return hipGetLastError();
+}
+hipError_t launch_batch_sens(const BatchMap &m, int nblocks, const DenseView &v, const AdjGroup &f,
+                             int cnt, hipStream_t s) {
+  hipLaunchKernelGGL(kb_sens, dim3(nblocks), dim3(256), 0, s, m, v.w, f, cnt);
+  return hipGetLastError();
 }
 
 hipError_t launch_batch_rows(const BatchMap &m, int nblocks, const DenseView &v, const double *Tn,

@@ -8,6 +8,8 @@ scaled together, so sum(M dJ/dM) + sum(g dJ/dg) = 0 (steps without sources).
 Each line solve has a relative error of a few 1e-15; six steps of three
 solves, forwards and backwards, stay below 1e-12 of the sums' magnitudes."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -97,6 +99,38 @@ def test_dense_steps_match_oracle_and_adjoint_identities(shape, strong):
     assert abs((p["G"] * h).sum() - (gT0 * p["T0"]).sum()) <= 1e-12 * size
     terms = [p["M"] * gM] + [a * b for a, b in zip(p["g"], (gz, gy, gx))]
     assert abs(sum(t.sum() for t in terms)) <= 1e-12 * sum(np.abs(t).sum() for t in terms)
+
+
+@pytest.mark.parametrize("every", [1, 3, 9])
+def test_gradients_do_not_depend_on_the_workspace(every):
+    """Sensitivities added four steps at a time and step by step (the smaller
+    workspace), with sources in neighbouring steps: the same bits."""
+    shape, steps, at = (9, 21, 35), 11, (0, 4, 5, 7)
+    p = _problem(shape, 0)
+    gp = _plan(p)
+    L = _lib.load()
+    n, s = int(np.prod(shape)), _lib.stream_handle()
+    rng = np.random.default_rng(every)
+    src = torch.from_numpy(rng.random((len(at),) + shape)).cuda()
+    G = torch.from_numpy(rng.random((steps,) + shape[1:])).cuda()
+    when = (ctypes.c_int32 * len(at))(*at)
+    T = torch.from_numpy(p["T0"]).cuda()
+    ckpt = torch.empty((-(-steps // every),) + shape, dtype=torch.float64, device="cuda")
+    _lib.check("hs2_grad_forward", L.hs2_grad_forward(
+        gp.plan, _lib.ptr(T), steps, every, _lib.ptr(ckpt), _lib.ptr(src), when, len(at), None, s))
+    got = []
+    for room in (L.hs2_grad_work_doubles(gp.plan, every), (3 * every + 6) * n):
+        work = torch.full((room,), np.nan, dtype=torch.float64, device="cuda")
+        out = [torch.full(shape, np.nan, dtype=torch.float64, device="cuda") for _ in range(5)]
+        out.append(torch.full_like(src, np.nan))
+        _lib.check("hs2_grad_backward", L.hs2_grad_backward(
+            gp.plan, steps, every, _lib.ptr(ckpt), _lib.ptr(src), when, len(at), _lib.ptr(G),
+            *[_lib.ptr(t) for t in out[:4]], _lib.ptr(out[5]), _lib.ptr(out[4]), _lib.ptr(work),
+            work.numel(), s))
+        torch.cuda.synchronize()
+        got.append(out)
+    assert all(torch.isfinite(a).all() for a in got[0])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
 def test_batched_edge_shapes_match_single_plans():
