@@ -130,8 +130,15 @@ def device():
     return torch.device("cuda", torch.cuda.current_device())
 
 
+# the handle by itself: a Stream object around it costs 2.8 us a call, of the 17
+# that a step of a small grid took
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if _raw_stream is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def ptr(t):

@@ -107,18 +107,20 @@ def _device_vmap(ADI_params, volumetric_elements):
 
 
 def _as_device_field(Tarray, shape):
-    dev = _lib.device()
     if isinstance(Tarray, torch.Tensor):
         if Tarray.dtype != torch.float64:
             raise ValueError("Tarray must be float64")
-        T = Tarray.to(dev).contiguous()
+        T = Tarray
+        if not T.is_cuda or T.get_device() != torch.cuda.current_device():
+            T = T.to(_lib.device())
+        T = T.contiguous()
         if T.data_ptr() % 16:
             T = T.clone()  # the kernels use 16-byte vector loads
         return T, True
     a = np.ascontiguousarray(Tarray, dtype=np.float64)
     if a.shape != tuple(shape):
         raise ValueError("Tarray shape %s does not match grid %s" % (a.shape, tuple(shape)))
-    return torch.from_numpy(a).to(dev), False
+    return torch.from_numpy(a).to(_lib.device()), False
 
 
 def run_adi_steps(ADI_params, ADI_steps, t, dt, Tarray, volumetric_elements, volumetric):
@@ -133,10 +135,10 @@ def run_adi_steps(ADI_params, ADI_steps, t, dt, Tarray, volumetric_elements, vol
     out = torch.empty_like(T)
     vmap = _device_vmap(ADI_params, volumetric_elements) if vtab is not None else None
     sf = torch.from_numpy(sfield).to(T.device) if sfield is not None else None
-    L = _lib.load()
-    _lib.check("hs2_step", L.hs2_step(ADI_params.plan, _lib.ptr(T), _lib.ptr(out), _lib.ptr(vmap),
-                                      _lib.host_ptr(vtab), 0 if vtab is None else len(vtab),
-                                      _lib.ptr(sf), None, _lib.stream_handle()))
+    # T and out are contiguous device tensors by now
+    _lib.check("hs2_step", _lib.load().hs2_step(
+        ADI_params.plan, T.data_ptr(), out.data_ptr(), _lib.ptr(vmap), _lib.host_ptr(vtab),
+        0 if vtab is None else len(vtab), _lib.ptr(sf), None, _lib.stream_handle()))
     if on_dev:
         return out
     return out.cpu().numpy()
