@@ -306,11 +306,6 @@ __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__
   extern __shared__ double lds[];
   __shared__ double2 carry[W > 1 ? 2 : 1][4];  // W > 1: the waves' carries, up and down
   double *vtab = lds + (size_t)t.nlds * NP * GL * 2;
-  for (int e = threadIdx.x; e < t.nlds * NP * GL; e += 256)
-    reinterpret_cast<double2 *>(lds)[e] = reinterpret_cast<const double2 *>(t.lane)[e];
-  if (SRC && vmap)
-    for (int e = threadIdx.x; e < kMaxVtab; e += 256) vtab[e] = vtab_g[e];
-  __syncthreads();
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int n = nx * ny * nz;
   const int lane = threadIdx.x & (kWave - 1);
@@ -318,7 +313,6 @@ __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__
   const int lig = lane % G + wr * kWave;  // lane of the row
   const int nj = (ny + LPW - 1) / LPW, units = nj * ((nz + KC - 1) / KC);
   const int unit = xcd_remap(blockIdx.x, gridDim.x) * RPB + wave / W;
-  if (W == 1 && unit >= units) return;  // W > 1: the block's waves meet at barriers
   const int uc = min(unit, units - 1);
   const int kc = uc / nj, jg = uc - kc * nj;
   const int jr = jg * LPW + lane / G;
@@ -342,6 +336,13 @@ __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__
   double Tm[CPL], T[CPL], Tp[CPL];
   load(k0 > 0 ? k0 - 1 : k0, j, Tm);
   load(k0, j, T);
+  // (behind the wave's own first loads: the two wait together)
+  for (int e = threadIdx.x; e < t.nlds * NP * GL; e += 256)
+    reinterpret_cast<double2 *>(lds)[e] = reinterpret_cast<const double2 *>(t.lane)[e];
+  if (SRC && vmap)
+    for (int e = threadIdx.x; e < kMaxVtab; e += 256) vtab[e] = vtab_g[e];
+  __syncthreads();
+  if (W == 1 && unit >= units) return;  // W > 1: the block's waves meet at barriers
   uint32_t erow = ~0u;
   double ex[kRowExpl];
   for (int kk = k0; kk < ke; kk++) {
