@@ -84,13 +84,21 @@ struct hs2_plan {
 
 enum { KIND_X2 = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, KIND_SENS = 5, NKIND = 6 };
 
+// Instances that run together: a range of blocks of every launch kind
+struct batch_group {
+  int maxsteps = 0;
+  int off[NKIND] = {}, nblk[NKIND] = {};
+  hipGraphExec_t fwd_exec = nullptr, bwd_exec = nullptr;
+  std::vector<const void *> fwd_key, bwd_key;
+};
+
 struct hs2_batch {
   int ninst = 0, K = 0, maxsteps = 0, device = 0;
   std::vector<hs2::BatchInst> inst;
   long long N = 0, H = 0, CK = 0;  // cells, history values, checkpoint values
   hs2::BatchInst *d_inst = nullptr;
   int *d_ctr = nullptr;
-  int nblk[NKIND] = {};
+  std::vector<batch_group> groups;
   int *d_blk_inst[NKIND] = {};
   int *d_blk0[NKIND] = {};
   hs2::DenseView dv{};
@@ -98,13 +106,7 @@ struct hs2_batch {
   int use_graph = 1, chunk = 8;
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
-  hipGraphExec_t fwd_exec = nullptr, bwd_exec = nullptr;
-  std::vector<const void *> fwd_key, bwd_key;
 };
-
-namespace {
-
-}  // namespace
 
 // Untuned y / z shape: segments of up to 16 cells (32-cell segments spill
 // registers), and blocks of about 256 threads, as the tuner picks at 256 and
@@ -324,8 +326,9 @@ void free_coefficients(hs2_plan *p) {
 // ------------------------------------------------------------- batches
 namespace {
 
-hs2::BatchMap batch_map(const hs2_batch *b, int kind, int rule, int j) {
-  return hs2::BatchMap{b->d_inst, b->d_blk_inst[kind], b->d_blk0[kind], b->d_ctr, rule, j, b->K};
+hs2::BatchMap batch_map(const hs2_batch *b, const batch_group &g, int kind, int rule, int j) {
+  return hs2::BatchMap{b->d_inst, b->d_blk_inst[kind], b->d_blk0[kind], b->d_ctr, rule, j, b->K,
+                       g.off[kind]};
 }
 
 int blocks_of(const hs2::BatchInst &I, int kind) {
@@ -342,8 +345,10 @@ int blocks_of(const hs2::BatchInst &I, int kind) {
 }
 
 void batch_free(hs2_batch *b) {
-  if (b->fwd_exec) (void)hipGraphExecDestroy(b->fwd_exec);
-  if (b->bwd_exec) (void)hipGraphExecDestroy(b->bwd_exec);
+  for (batch_group &g : b->groups) {
+    if (g.fwd_exec) (void)hipGraphExecDestroy(g.fwd_exec);
+    if (g.bwd_exec) (void)hipGraphExecDestroy(g.bwd_exec);
+  }
   if (b->ev_in) (void)hipEventDestroy(b->ev_in);
   if (b->ev_out) (void)hipEventDestroy(b->ev_out);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -375,42 +380,42 @@ BatchWork batch_work(const hs2_batch *b, double *w) {
 }
 
 // forward: `steps` steps (ckpt store, x, y, z with the readout, tick)
-hipError_t emit_forward(hs2_batch *b, double *T, const double *src, double *hist,
+hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const double *src, double *hist,
                         const BatchWork &w, int steps, hipStream_t s) {
   hipError_t e = hipSuccess;
   for (int c = 0; c < steps && e == hipSuccess; c++) {
-    e = hs2::launch_batch_rows(batch_map(b, KIND_X2, hs2::RULE_FWD, 0), b->nblk[KIND_X2], b->dv,
+    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X2, hs2::RULE_FWD, c), g.nblk[KIND_X2], b->dv,
                                T, w.ws, src, w.ck, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, KIND_Y, hs2::RULE_FWD, 0), b->nblk[KIND_Y], 1, b->dv,
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Y, hs2::RULE_FWD, c), g.nblk[KIND_Y], 1, b->dv,
                                  T, w.ws, w.ws, nullptr, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, KIND_Z, hs2::RULE_FWD, 0), b->nblk[KIND_Z], 0, b->dv,
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Z, hs2::RULE_FWD, c), g.nblk[KIND_Z], 0, b->dv,
                                  T, w.ws, T, hist, false, s);
-    if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 0, 1, 1, s);
   }
+  if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 0, steps, 1, s);
   return e;
 }
 
 // one backward segment: load checkpoints, recompute its K steps keeping every
 // state, K adjoint steps, tick
-hipError_t emit_backward_segment(hs2_batch *b, const double *src, const double *ghist,
+hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const double *src, const double *ghist,
                                  double *gM, double *gz, double *gy, double *gx, double *gsrc,
                                  const BatchWork &w, hipStream_t s) {
   const int K = b->K;
   const size_t N = (size_t)b->N;
-  hipError_t e = hs2::launch_batch_ckpt_load(batch_map(b, KIND_CELL, hs2::RULE_SEG, 0),
-                                             b->nblk[KIND_CELL], w.ck, w.seg, b->N, s);
+  hipError_t e = hs2::launch_batch_ckpt_load(batch_map(b, g, KIND_CELL, hs2::RULE_SEG, 0),
+                                             g.nblk[KIND_CELL], w.ck, w.seg, b->N, s);
   for (int j = 0; j < K && e == hipSuccess; j++) {
     const double *in = w.seg + (size_t)j * N;
     double *tx = w.segx + (size_t)j * N, *ty = w.segy + (size_t)j * N;
-    e = hs2::launch_batch_rows(batch_map(b, KIND_X2, hs2::RULE_RECOMP, j), b->nblk[KIND_X2], b->dv,
+    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X2, hs2::RULE_RECOMP, j), g.nblk[KIND_X2], b->dv,
                                in, tx, src, nullptr, false, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, KIND_Y, hs2::RULE_RECOMP, j), b->nblk[KIND_Y], 1,
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Y, hs2::RULE_RECOMP, j), g.nblk[KIND_Y], 1,
                                  b->dv, in, tx, ty, nullptr, false, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, KIND_Z, hs2::RULE_RECOMP, j), b->nblk[KIND_Z], 0,
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Z, hs2::RULE_RECOMP, j), g.nblk[KIND_Z], 0,
                                  b->dv, in, ty, w.seg + (size_t)(j + 1) * N, nullptr, false, s);
   }
   // adjoint steps, latest first: lambda from the solves of the step after (the
@@ -420,13 +425,13 @@ hipError_t emit_backward_segment(hs2_batch *b, const double *src, const double *
   for (int j = 0; j < K && e == hipSuccess; j++) {
     double *uz = w.u + (size_t)(j % S) * 3 * N, *uy = uz + N, *ux = uy + N;
     const double *after = w.u + (size_t)((j > 0 ? j - 1 : K - 1) % S) * 3 * N;
-    e = hs2::launch_batch_lambda(batch_map(b, KIND_Z, hs2::RULE_BWD, j), b->nblk[KIND_Z], b->dv,
+    e = hs2::launch_batch_lambda(batch_map(b, g, KIND_Z, hs2::RULE_BWD, j), g.nblk[KIND_Z], b->dv,
                                  after, b->N, ghist, uz, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_adj_line(batch_map(b, KIND_Y, hs2::RULE_BWD, j), b->nblk[KIND_Y], 1,
+      e = hs2::launch_batch_adj_line(batch_map(b, g, KIND_Y, hs2::RULE_BWD, j), g.nblk[KIND_Y], 1,
                                      b->dv, uz, 1, uy, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_adj_line(batch_map(b, KIND_AX, hs2::RULE_BWD, j), b->nblk[KIND_AX], 2,
+      e = hs2::launch_batch_adj_line(batch_map(b, g, KIND_AX, hs2::RULE_BWD, j), g.nblk[KIND_AX], 2,
                                      b->dv, uy, 1, ux, s);
     if (e == hipSuccess && (j % S == S - 1 || j == K - 1)) {
       const int j0 = j - j % S;
@@ -438,7 +443,7 @@ hipError_t emit_backward_segment(hs2_batch *b, const double *src, const double *
       f.gg[0] = gz; f.gg[1] = gy; f.gg[2] = gx;
       for (double *&gs : f.gsrc) gs = gsrc;
       f.N = b->N;
-      e = hs2::launch_batch_sens(batch_map(b, KIND_SENS, hs2::RULE_BWD, j0), b->nblk[KIND_SENS],
+      e = hs2::launch_batch_sens(batch_map(b, g, KIND_SENS, hs2::RULE_BWD, j0), g.nblk[KIND_SENS],
                                  b->dv, f, j - j0 + 1, s);
     }
   }
@@ -1408,18 +1413,37 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
   if (rc == HS2_OK)
     bad(hipMemcpy(b->d_inst, b->inst.data(), sizeof(hs2::BatchInst) * ninst,
                   hipMemcpyHostToDevice), "hipMemcpy");
+  // groups of about kBatchGroupCells cells, instances of like step counts together
+  std::vector<int> order(ninst);
+  for (int i = 0; i < ninst; i++) order[i] = i;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int x, int y) { return b->inst[x].nsteps < b->inst[y].nsteps; });
+  const long long ngroup =
+      std::max<long long>(1, (off + hs2::kBatchGroupCells / 2) / hs2::kBatchGroupCells);
+  std::vector<int> group(ninst);
+  long long before = 0;
+  for (int i : order) {  // by the middle of the instance's cells
+    const long long n = (long long)b->inst[i].nz * b->inst[i].ny * b->inst[i].nx;
+    group[i] = (int)std::min(ngroup - 1, (before + n / 2) * ngroup / off);
+    before += n;
+  }
+  b->groups.resize((size_t)ngroup);
+  for (int i : order)
+    b->groups[group[i]].maxsteps = std::max(b->groups[group[i]].maxsteps, b->inst[i].nsteps);
   for (int k = 0; k < NKIND && rc == HS2_OK; k++) {
-    std::vector<int> b0(ninst + 1, 0), owner;
-    for (int i = 0; i < ninst; i++) {
+    std::vector<int> b0(ninst, 0), owner;
+    for (int i : order) {
+      batch_group &g = b->groups[group[i]];
       const int nb = blocks_of(b->inst[i], k);
-      b0[i + 1] = b0[i] + nb;
+      if (!g.nblk[k]) g.off[k] = (int)owner.size();
+      g.nblk[k] += nb;
+      b0[i] = (int)owner.size();
       owner.insert(owner.end(), nb, i);
     }
-    b->nblk[k] = b0[ninst];
-    bad(hipMalloc(&b->d_blk0[k], sizeof(int) * (ninst + 1)), "hipMalloc");
+    bad(hipMalloc(&b->d_blk0[k], sizeof(int) * ninst), "hipMalloc");
     bad(hipMalloc(&b->d_blk_inst[k], sizeof(int) * owner.size()), "hipMalloc");
     if (rc == HS2_OK) {
-      bad(hipMemcpy(b->d_blk0[k], b0.data(), sizeof(int) * (ninst + 1), hipMemcpyHostToDevice),
+      bad(hipMemcpy(b->d_blk0[k], b0.data(), sizeof(int) * ninst, hipMemcpyHostToDevice),
           "hipMemcpy");
       bad(hipMemcpy(b->d_blk_inst[k], owner.data(), sizeof(int) * owner.size(),
                     hipMemcpyHostToDevice), "hipMemcpy");
@@ -1496,16 +1520,20 @@ int hs2_batch_forward(hs2_batch *b, double *d_T, const double *d_src, double *d_
   const BatchWork w = batch_work(b, d_work);
   HIP_TRY(hipEventRecord(b->ev_in, (hipStream_t)stream));
   HIP_TRY(hipStreamWaitEvent(b->stream, b->ev_in, 0));
-  HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 0, 0, 0, b->stream));
-  const int C = std::min(b->chunk, b->maxsteps);
-  const int reps = (b->maxsteps + C - 1) / C;
-  const std::vector<const void *> key = {d_T, d_src, d_hist, d_work, b->dv.M, b->dv.w,
-                                         b->dv.g[0], b->dv.g[1], b->dv.g[2],
-                                         (const void *)(intptr_t)C};
-  const int rc = batch_replay(b, &b->fwd_exec, &b->fwd_key, key, reps,
-                              [&](hipStream_t s) { return emit_forward(b, d_T, d_src, d_hist, w, C, s); },
-                              "hs2_batch_forward");
-  if (rc != HS2_OK) return rc;
+  for (batch_group &g : b->groups) {
+    if (!g.maxsteps) continue;
+    HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 0, 0, 0, b->stream));
+    const int C = std::min(b->chunk, g.maxsteps);
+    const int reps = (g.maxsteps + C - 1) / C;
+    const std::vector<const void *> key = {d_T, d_src, d_hist, d_work, b->dv.M, b->dv.w,
+                                           b->dv.g[0], b->dv.g[1], b->dv.g[2],
+                                           (const void *)(intptr_t)C};
+    const int rc = batch_replay(
+        b, &g.fwd_exec, &g.fwd_key, key, reps,
+        [&](hipStream_t s) { return emit_forward(b, g, d_T, d_src, d_hist, w, C, s); },
+        "hs2_batch_forward");
+    if (rc != HS2_OK) return rc;
+  }
   HIP_TRY(hipEventRecord(b->ev_out, b->stream));
   HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
   return HS2_OK;
@@ -1528,18 +1556,22 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   HIP_TRY(hs2::launch_fill(d_gy, b->N, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gx, b->N, 0.0, s));
   if (d_gsrc) HIP_TRY(hs2::launch_fill(d_gsrc, b->N, 0.0, s));
-  HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 1, 0, 0, s));
-  const int reps = (b->maxsteps + b->K - 1) / b->K;
   const std::vector<const void *> key = {d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc,
                                          d_work, b->dv.M, b->dv.w, b->dv.g[0], b->dv.g[1],
                                          b->dv.g[2]};
-  const int rc = batch_replay(
-      b, &b->bwd_exec, &b->bwd_key, key, reps,
-      [&](hipStream_t st) {
-        return emit_backward_segment(b, d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc, w, st);
-      },
-      "hs2_batch_backward");
-  if (rc != HS2_OK) return rc;
+  for (batch_group &g : b->groups) {
+    if (!g.maxsteps) continue;
+    HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 1, 0, 0, s));
+    const int reps = (g.maxsteps + b->K - 1) / b->K;
+    const int rc = batch_replay(
+        b, &g.bwd_exec, &g.bwd_key, key, reps,
+        [&](hipStream_t st) {
+          return emit_backward_segment(b, g, d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc, w,
+                                       st);
+        },
+        "hs2_batch_backward");
+    if (rc != HS2_OK) return rc;
+  }
   HIP_TRY(hipEventRecord(b->ev_out, s));
   HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
   return HS2_OK;

@@ -1,12 +1,13 @@
 // Batched execution of many independent ADI problems of different sizes and
-// step counts: one launch per sweep covers every instance.  Each launch kind
+// step counts: one launch per sweep covers every instance of a group (the
+// groups run one after another; see kBatchGroupCells).  Each launch kind
 // has a block -> instance table; a block finds its instance, its local block
 // index and its instance's current step, and works on that instance's slice
 // of the concatenated fields (per-voxel coefficients, DenseView).
 //
-// Time is driven by counters in device memory (ctr[0]: forward step,
-// ctr[1]: backward segment), so a captured graph of a chunk of steps can be
-// replayed without changing any kernel argument.  Checkpoints are aligned
+// Time is driven by counters in device memory (ctr[0]: the forward step a
+// chunk of steps begins with, ctr[1]: backward segment), so a captured graph
+// of a chunk can be replayed without changing any kernel argument.  Checkpoints are aligned
 // to each instance's end: with K steps per segment, backward segment s of
 // instance i covers steps [max(0, e-K), e), e = nsteps_i - s*K, so every
 // instance is at the same position inside its segment and the recomputation
@@ -25,6 +26,14 @@ constexpr int kBatchWaves = 4;     // waves (units of rows) per block of the x k
 constexpr int kBatchSeg = 8;       // cells per thread segment of the line kernels
 constexpr int kBatchPlanes = 2;    // planes a wave of the x sweep walks (1, 4: 2% slower, 8: 18%)
 constexpr int kBatchSensPlanes = 8;  // planes per block of the sensitivity pass
+// Cells of a group, about: a step's fields (T, T*, M, three conductances, w: 49
+// bytes a cell) then fit the 256 MB Infinity Cache, and launches stay long.
+// ns per cell and step by the cells run together, forward | with gradient:
+// 12.7 million 0.0265 | 0.1023, 8.7 0.0259 | 0.1013, 4.2 to 4.8 0.0241 | 0.0953,
+// 3.3 0.0261, 2.6 0.1029, 2.0 0.0305.  24 instances of 32..128^3 and 40 to 160
+// steps: histories 29.7 -> 28.0 ms (0.6 of it one counter launch a chunk instead
+// of one a step), gradients 118.1 -> 113.1.
+constexpr long long kBatchGroupCells = 4500000;
 constexpr int kBatchAlign = 32;    // instance offsets are multiples of this many cells
 
 // Segments of kBatchSeg cells per line of L cells in the y and z line
@@ -60,6 +69,7 @@ struct BatchMap {
   const int *blk0;      // first block of each instance
   const int *ctr;       // device counters
   int rule, j, K;
+  int off;              // first block of the launch's group in the tables
 };
 
 // Logical block of hardware block b among nb.  Hardware hands block b to XCD
@@ -78,7 +88,7 @@ __device__ __forceinline__ int batch_block(int b, int nb) {
 // Instance, local block and step of this block; false if the instance has
 // nothing to do under the launch's rule (the whole block returns).
 __device__ __forceinline__ bool batch_locate(const BatchMap &m, BatchInst &I, int &local, int &t) {
-  const int gb = batch_block(blockIdx.x, gridDim.x);
+  const int gb = m.off + batch_block(blockIdx.x, gridDim.x);
   const int i = m.blk_inst[gb];
   local = gb - m.blk0[i];
   I = m.inst[i];
@@ -87,7 +97,7 @@ __device__ __forceinline__ bool batch_locate(const BatchMap &m, BatchInst &I, in
     return true;
   }
   if (m.rule == RULE_FWD) {
-    t = m.ctr[0];
+    t = m.ctr[0] + m.j;
     return t < I.nsteps;
   }
   const int e = I.nsteps - m.ctr[1] * m.K;
