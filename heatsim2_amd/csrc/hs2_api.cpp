@@ -11,6 +11,7 @@
 #include <string>
 #include <tuple>
 #include <unordered_map>
+#include <mutex>
 #include <vector>
 
 #include "../../include/heatsim2_amd.h"
@@ -78,6 +79,11 @@ struct hs2_plan {
   double *d_vsteps = nullptr;   // per-step source tables (hs2_run)
   size_t vsteps_cap = 0;        // doubles
   int *d_check = nullptr;       // per-block maxima of the maps (validation)
+  // second stream of hs2_grad_backward (made by its first call that has use for
+  // it); a call that finds it taken by another thread's does without
+  std::mutex aux_mu;
+  hipStream_t aux = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hs2::XConfig xcfg{0, 0, 0};
   hs2::SConfig scfg[2] = {{0, 0}, {0, 0}};  // [0] z, [1] y
 };
@@ -276,6 +282,35 @@ hipError_t adj_stencil(const hs2_plan *p, const hs2::AdjFields &f, hipStream_t s
 // sensitivities of kAdjGroup steps in one pass)
 bool grad_grouped(const hs2_plan *p) {
   return p->mode == MODE_DENSE && hs2::dense_cols_ok(grid_of(p), 0);
+}
+
+// hs2_grad_backward recomputes the segment before on a second stream while a
+// segment's adjoint steps run, on grids of up to this many cells: the launches
+// of one fill the ramps and waits of the other's.  us per step of a backward
+// pass, one stream | two: 29x45x51 33.6 | 26.9, 48x64x64 35.7 | 27.5, 64x128x128
+// 75.6 | 68.6, 100x128x160 156 | 146, 128x160x160 231 | 221, 160x200x200 481 |
+// 469: beyond, 2% is not worth a second store of states.
+constexpr size_t kOverlapCells = 4000000;
+bool grad_overlaps(const hs2_plan *p) { return grad_grouped(p) && (size_t)p->n <= kOverlapCells; }
+
+// the second stream is there and `s` is not being captured
+bool aux_stream(hs2_plan *p, hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
+  if (p->aux) return true;
+  if (!p->ev_fork && hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming) != hipSuccess) {
+    p->ev_fork = nullptr;
+    return false;
+  }
+  if (!p->ev_join && hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming) != hipSuccess) {
+    p->ev_join = nullptr;
+    return false;
+  }
+  if (hipStreamCreateWithFlags(&p->aux, hipStreamNonBlocking) != hipSuccess) {
+    p->aux = nullptr;
+    return false;
+  }
+  return true;
 }
 
 // step -> source index (-1: none); validates the schedule
@@ -807,6 +842,9 @@ void hs2_plan_destroy(hs2_plan *p) {
   (void)hipFree(p->d_vtab);
   (void)hipFree(p->d_vsteps);
   (void)hipFree(p->d_check);
+  if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
+  if (p->ev_join) (void)hipEventDestroy(p->ev_join);
+  if (p->aux) (void)hipStreamDestroy(p->aux);
   delete p;
 }
 
@@ -1227,7 +1265,9 @@ int hs2_run_timed(hs2_plan *p, double *d_T, int nsteps, int method, double *kern
 
 size_t hs2_grad_work_doubles(const hs2_plan *p, int ckpt_every) {
   if (!p || ckpt_every < 1) return 0;
-  return (3 * (size_t)ckpt_every + (grad_grouped(p) ? 1 + 3 * hs2::kAdjGroup : 6)) * (size_t)p->n;
+  const size_t K = (size_t)ckpt_every, n = (size_t)p->n;
+  if (!grad_grouped(p)) return (3 * K + 6) * n;
+  return ((grad_overlaps(p) ? 2 : 1) * (3 * K + 1) + 3 * hs2::kAdjGroup) * n;
 }
 
 int hs2_grad_forward(hs2_plan *p, double *d_T, int nsteps, int ckpt_every, double *d_ckpt,
@@ -1286,16 +1326,22 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
   const size_t n = (size_t)p->n, nyx = (size_t)g.ny * g.nx;
   const int K = ckpt_every;
   // segment store: T^{n0} .. T^{n0+K} (K+1 fields), and T*, T** of each of
-  // its K steps, so every state of the segment is computed once
-  double *seg = d_work;
-  double *segx = seg + (size_t)(K + 1) * n, *segy = segx + (size_t)K * n;
+  // its K steps, so every state of the segment is computed once; with two of
+  // them the segment before is recomputed while this one's adjoint steps run
+  const int nseg = (nsteps + K - 1) / K;
+  const size_t store = 3 * (size_t)K + 1;  // fields
+  const bool grouped = grad_grouped(p);
+  std::unique_lock<std::mutex> aux_lock(p->aux_mu, std::defer_lock);
+  const bool overlap = grad_overlaps(p) && nseg > 1 &&
+                       work_doubles / n >= 2 * store + 3 * hs2::kAdjGroup &&
+                       aux_lock.try_lock() && aux_stream(p, s);
+  const size_t stores = overlap ? 2 : 1;
   // per-voxel coefficients: the solves of a group of steps; class maps: u_x,
   // u_y, u_z of one step, lambda and the next lambda
-  double *u = segy + (size_t)K * n;
+  double *u = d_work + stores * store * n;
   double *ux = u, *uy = ux + n, *uz = uy + n, *lam = uz + n, *lam2 = lam + n;
-  const bool grouped = grad_grouped(p);
   // steps of a group: as many as the workspace has room for (at least one)
-  const int S = (int)std::min<size_t>(hs2::kAdjGroup, (work_doubles / n - (3 * (size_t)K + 1)) / 3);
+  const int S = (int)std::min<size_t>(hs2::kAdjGroup, (work_doubles / n - stores * store) / 3);
   const double *after = nullptr;  // grouped: the solves of the step after
   HIP_TRY(hs2::launch_fill(d_gM, n, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gz, n, 0.0, s));
@@ -1303,27 +1349,33 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
   HIP_TRY(hs2::launch_fill(d_gx, n, 0.0, s));
   if (!grouped)
     HIP_TRY(hs2::launch_lam_from_readout(g, d_grad_hist + (size_t)(nsteps - 1) * nyx, lam, s));
-  const int nseg = (nsteps + K - 1) / K;
-  for (int sg = nseg - 1; sg >= 0; sg--) {
-    const int n0 = sg * K, n1 = std::min(nsteps, n0 + K);
-    HIP_TRY(hipMemcpyAsync(seg, d_ckpt + (size_t)sg * n, n * sizeof(double),
-                           hipMemcpyDeviceToDevice, s));
-    for (int t = n0; t < n1; t++) {  // recompute the segment's states
-      const size_t q = (size_t)(t - n0);
-      const double *sf = src[t] >= 0 ? d_src + (size_t)src[t] * n : nullptr;
-      rc = step_states(p, seg + q * n, segx + q * n, segy + q * n, seg + (q + 1) * n, sf,
-                       nullptr, s);
-      if (rc != HS2_OK) return rc;
-    }
-    for (int t = n1 - 1; grouped && t >= n0; t--) {
+  auto seg_of = [&](int sg) { return d_work + (overlap ? (size_t)(sg & 1) : 0) * store * n; };
+
+  // step i of segment sg: the states it leaves
+  auto recompute = [&](int sg, int i, hipStream_t st) -> int {
+    double *seg = seg_of(sg), *segx = seg + (size_t)(K + 1) * n, *segy = segx + (size_t)K * n;
+    const size_t q = (size_t)i;
+    if (i == 0)
+      HIP_TRY(hipMemcpyAsync(seg, d_ckpt + (size_t)sg * n, n * sizeof(double),
+                             hipMemcpyDeviceToDevice, st));
+    const int t = sg * K + i;
+    const double *sf = src[t] >= 0 ? d_src + (size_t)src[t] * n : nullptr;
+    return step_states(p, seg + q * n, segx + q * n, segy + q * n, seg + (q + 1) * n, sf, nullptr,
+                       st);
+  };
+  // adjoint step t of segment sg (steps n0 .. n1 - 1)
+  auto adjoint = [&](int sg, int n0, int n1, int t) -> int {
+    double *seg = seg_of(sg), *segx = seg + (size_t)(K + 1) * n, *segy = segx + (size_t)K * n;
+    if (grouped) {
       const int slot = (n1 - 1 - t) % S;
       double *wz = u + (size_t)slot * 3 * n, *wy = wz + n, *wx = wy + n;
       HIP_TRY(hs2::launch_dense_lambda(g, p->dv, after ? after + 2 * n : nullptr,
-                                       after ? after + n : nullptr, after, d_grad_hist + (size_t)t * nyx, true, wz, s));
+                                       after ? after + n : nullptr, after,
+                                       d_grad_hist + (size_t)t * nyx, true, wz, s));
       HIP_TRY(adj_line(p, 1, wz, 1, wy, s));
       HIP_TRY(adj_line(p, 2, wy, 1, wx, s));
       after = wz;
-      if (slot < S - 1 && t > n0) continue;
+      if (slot < S - 1 && t > n0) return HS2_OK;
       const size_t q = (size_t)(t + slot - n0);  // the group's latest step
       hs2::AdjGroup f{};
       f.T = seg + q * n; f.Tx = segx + q * n; f.Ty = segy + q * n;
@@ -1336,22 +1388,53 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
       }
       f.N = (long long)n;
       HIP_TRY(hs2::launch_dense_sens(g, p->dv, f, slot + 1, s));
+      return HS2_OK;
     }
-    for (int t = n1 - 1; !grouped && t >= n0; t--) {
-      const size_t q = (size_t)(t - n0);
-      HIP_TRY(adj_line(p, 0, lam, 0, uz, s));
-      HIP_TRY(adj_line(p, 1, uz, 1, uy, s));
-      HIP_TRY(adj_line(p, 2, uy, 1, ux, s));
-      hs2::AdjFields f{};
-      f.Tn = seg + q * n; f.Tx = segx + q * n; f.Ty = segy + q * n; f.Tn1 = seg + (q + 1) * n;
-      f.ux = ux; f.uy = uy; f.uz = uz;
-      f.ghist = t >= 1 ? d_grad_hist + (size_t)(t - 1) * nyx : nullptr;
-      f.lam_out = lam2;
-      f.gM = d_gM;
-      f.gg[0] = d_gz; f.gg[1] = d_gy; f.gg[2] = d_gx;
-      f.gsrc = src[t] >= 0 ? d_gsrc + (size_t)src[t] * n : nullptr;
-      HIP_TRY(adj_stencil(p, f, s));
-      std::swap(lam, lam2);
+    const size_t q = (size_t)(t - n0);
+    HIP_TRY(adj_line(p, 0, lam, 0, uz, s));
+    HIP_TRY(adj_line(p, 1, uz, 1, uy, s));
+    HIP_TRY(adj_line(p, 2, uy, 1, ux, s));
+    hs2::AdjFields f{};
+    f.Tn = seg + q * n; f.Tx = segx + q * n; f.Ty = segy + q * n; f.Tn1 = seg + (q + 1) * n;
+    f.ux = ux; f.uy = uy; f.uz = uz;
+    f.ghist = t >= 1 ? d_grad_hist + (size_t)(t - 1) * nyx : nullptr;
+    f.lam_out = lam2;
+    f.gM = d_gM;
+    f.gg[0] = d_gz; f.gg[1] = d_gy; f.gg[2] = d_gx;
+    f.gsrc = src[t] >= 0 ? d_gsrc + (size_t)src[t] * n : nullptr;
+    HIP_TRY(adj_stencil(p, f, s));
+    std::swap(lam, lam2);
+    return HS2_OK;
+  };
+  // whatever happens after the second stream was given work, it has ended or
+  // `s` waits for it when this call returns
+  struct Joined {
+    hipStream_t aux = nullptr;
+    ~Joined() {
+      if (aux) (void)hipStreamSynchronize(aux);
+    }
+  } pending;
+  for (int i = 0; i < nsteps - (nseg - 1) * K; i++)
+    if ((rc = recompute(nseg - 1, i, s)) != HS2_OK) return rc;
+  for (int sg = nseg - 1; sg >= 0; sg--) {
+    const int n0 = sg * K, n1 = std::min(nsteps, n0 + K);
+    const bool fork = overlap && sg > 0;
+    if (fork) {  // its store was read by the adjoint steps of segment sg + 1
+      HIP_TRY(hipEventRecord(p->ev_fork, s));
+      HIP_TRY(hipStreamWaitEvent(p->aux, p->ev_fork, 0));
+      pending.aux = p->aux;
+    }
+    for (int i = 0; i < (fork ? K : n1 - n0); i++) {  // in turn: both streams get work at once
+      if (fork && (rc = recompute(sg - 1, i, p->aux)) != HS2_OK) return rc;
+      if (i < n1 - n0 && (rc = adjoint(sg, n0, n1, n1 - 1 - i)) != HS2_OK) return rc;
+    }
+    if (fork) {
+      HIP_TRY(hipEventRecord(p->ev_join, p->aux));
+      HIP_TRY(hipStreamWaitEvent(s, p->ev_join, 0));
+      pending.aux = nullptr;
+    } else {
+      for (int i = 0; sg > 0 && i < K; i++)
+        if ((rc = recompute(sg - 1, i, s)) != HS2_OK) return rc;
     }
   }
   if (d_gT0 && grouped)

@@ -199,10 +199,12 @@ int hs2_run_timed(hs2_plan *plan, double *d_T, int nsteps, int method, double *k
  * respect to per-voxel parameters need hs2_plan_set_dense. */
 
 /* Doubles of device workspace for hs2_grad_backward: (3*ckpt_every+6)*n (each
- * segment's states T^n, T*, T** are recomputed once and kept), and 7*n more on
- * per-voxel coefficients, where sensitivities are added for four steps at a
- * time; hs2_grad_backward also takes the smaller one and then adds them step
- * by step, with the same results. */
+ * segment's states T^n, T*, T** are recomputed once and kept) on class maps.
+ * On per-voxel coefficients 7*n more, where sensitivities are added for four
+ * steps at a time, and on small grids another (3*ckpt_every+1)*n, with which a
+ * segment is recomputed on a second stream beside the adjoint steps of the one
+ * after it.  hs2_grad_backward also takes the smaller ones and then does
+ * without, with the same results. */
 size_t hs2_grad_work_doubles(const hs2_plan *plan, int ckpt_every);
 
 /* Forward pass: nsteps steps in place on d_T (T^0 in, T^nsteps out),
