@@ -90,9 +90,13 @@ struct hs2_plan {
 
 enum { KIND_X2 = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, KIND_SENS = 5, NKIND = 6 };
 
-// Instances that run together: a range of blocks of every launch kind
+// Instances that run together: a range of blocks of every launch kind.  The
+// groups of a lane run one after another on the lane's stream, on its two
+// counters.
+constexpr int kBatchLanes = 2;
 struct batch_group {
-  int maxsteps = 0;
+  int maxsteps = 0, lane = 0;
+  long long work = 0;  // cells x steps
   int off[NKIND] = {}, nblk[NKIND] = {};
   hipGraphExec_t fwd_exec = nullptr, bwd_exec = nullptr;
   std::vector<const void *> fwd_key, bwd_key;
@@ -110,8 +114,8 @@ struct hs2_batch {
   hs2::DenseView dv{};
   bool have_coef = false;
   int use_graph = 1, chunk = 8;
-  hipStream_t stream = nullptr;
-  hipEvent_t ev_in = nullptr, ev_out = nullptr;
+  hipStream_t stream[kBatchLanes] = {};  // [1]: where there is more than one group
+  hipEvent_t ev_in = nullptr, ev_out = nullptr, ev_lane = nullptr;
 };
 
 // Untuned y / z shape: segments of up to 16 cells (32-cell segments spill
@@ -362,7 +366,8 @@ void free_coefficients(hs2_plan *p) {
 namespace {
 
 hs2::BatchMap batch_map(const hs2_batch *b, const batch_group &g, int kind, int rule, int j) {
-  return hs2::BatchMap{b->d_inst, b->d_blk_inst[kind], b->d_blk0[kind], b->d_ctr, rule, j, b->K,
+  return hs2::BatchMap{b->d_inst, b->d_blk_inst[kind], b->d_blk0[kind],
+                       b->d_ctr + 2 * g.lane, rule, j, b->K,
                        g.off[kind]};
 }
 
@@ -386,7 +391,9 @@ void batch_free(hs2_batch *b) {
   }
   if (b->ev_in) (void)hipEventDestroy(b->ev_in);
   if (b->ev_out) (void)hipEventDestroy(b->ev_out);
-  if (b->stream) (void)hipStreamDestroy(b->stream);
+  if (b->ev_lane) (void)hipEventDestroy(b->ev_lane);
+  for (hipStream_t st : b->stream)
+    if (st) (void)hipStreamDestroy(st);
   (void)hipFree(b->d_inst);
   (void)hipFree(b->d_ctr);
   for (int k = 0; k < NKIND; k++) {
@@ -428,7 +435,7 @@ hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const dou
       e = hs2::launch_batch_cols(batch_map(b, g, KIND_Z, hs2::RULE_FWD, c), g.nblk[KIND_Z], 0, b->dv,
                                  T, w.ws, T, hist, false, s);
   }
-  if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 0, steps, 1, s);
+  if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr + 2 * g.lane, 0, steps, 1, s);
   return e;
 }
 
@@ -482,17 +489,16 @@ hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const doubl
                                  b->dv, f, j - j0 + 1, s);
     }
   }
-  if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr, 1, 1, 1, s);
+  if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr + 2 * g.lane, 1, 1, 1, s);
   return e;
 }
 
-// run `emit` `reps` times on b->stream, through a graph captured once per key
+// one `emit` on `s`, through a graph captured once per key
 template <class Emit>
-int batch_replay(hs2_batch *b, hipGraphExec_t *exec, std::vector<const void *> *key,
-                 const std::vector<const void *> &want, int reps, Emit emit, const char *who) {
-  hipStream_t s = b->stream;
+int batch_replay(hs2_batch *b, hipStream_t s, hipGraphExec_t *exec, std::vector<const void *> *key,
+                 const std::vector<const void *> &want, Emit emit, const char *who) {
   if (!b->use_graph) {
-    for (int r = 0; r < reps; r++) HIP_TRY(emit(s));
+    HIP_TRY(emit(s));
     return HS2_OK;
   }
   if (!*exec || *key != want) {
@@ -517,7 +523,43 @@ int batch_replay(hs2_batch *b, hipGraphExec_t *exec, std::vector<const void *> *
     }
     *key = want;
   }
-  for (int r = 0; r < reps; r++) HIP_TRY(hipGraphLaunch(*exec, s));
+  HIP_TRY(hipGraphLaunch(*exec, s));
+  return HS2_OK;
+}
+
+// Every group's turns on its lane's stream, the lanes in turn so that all of
+// them have work at once; then the first lane waits for the others.  reset:
+// the counter that a group starts from 0; turns(g), turn(g).
+template <class Turns, class Turn>
+int batch_lanes(hs2_batch *b, int reset, Turns turns, Turn turn) {
+  size_t at[kBatchLanes] = {};
+  int done[kBatchLanes] = {};
+  for (int lane = 1; lane < kBatchLanes; lane++)
+    if (b->stream[lane]) HIP_TRY(hipStreamWaitEvent(b->stream[lane], b->ev_lane, 0));
+  for (bool any = true; any;) {
+    any = false;
+    for (int lane = 0; lane < kBatchLanes; lane++) {
+      while (at[lane] < b->groups.size() &&
+             (b->groups[at[lane]].lane != lane || !b->groups[at[lane]].maxsteps))
+        at[lane]++;
+      if (at[lane] == b->groups.size()) continue;
+      any = true;
+      batch_group &g = b->groups[at[lane]];
+      if (done[lane] == 0)
+        HIP_TRY(hs2::launch_batch_counter(b->d_ctr + 2 * lane, reset, 0, 0, b->stream[lane]));
+      const int rc = turn(g, b->stream[lane]);
+      if (rc != HS2_OK) return rc;
+      if (++done[lane] == turns(g)) {
+        done[lane] = 0;
+        at[lane]++;
+      }
+    }
+  }
+  for (int lane = 1; lane < kBatchLanes; lane++)
+    if (b->stream[lane]) {
+      HIP_TRY(hipEventRecord(b->ev_lane, b->stream[lane]));
+      HIP_TRY(hipStreamWaitEvent(b->stream[0], b->ev_lane, 0));
+    }
   return HS2_OK;
 }
 
@@ -1492,7 +1534,7 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
   };
   bad(hipGetDevice(&b->device), "hipGetDevice");
   bad(hipMalloc(&b->d_inst, sizeof(hs2::BatchInst) * ninst), "hipMalloc");
-  bad(hipMalloc(&b->d_ctr, 2 * sizeof(int)), "hipMalloc");
+  bad(hipMalloc(&b->d_ctr, 2 * kBatchLanes * sizeof(int)), "hipMalloc");
   if (rc == HS2_OK)
     bad(hipMemcpy(b->d_inst, b->inst.data(), sizeof(hs2::BatchInst) * ninst,
                   hipMemcpyHostToDevice), "hipMemcpy");
@@ -1502,7 +1544,8 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
   std::stable_sort(order.begin(), order.end(),
                    [&](int x, int y) { return b->inst[x].nsteps < b->inst[y].nsteps; });
   const long long ngroup =
-      std::max<long long>(1, (off + hs2::kBatchGroupCells / 2) / hs2::kBatchGroupCells);
+      std::max<long long>(std::min(ninst, kBatchLanes),
+                          (off + hs2::kBatchGroupCells / 2) / hs2::kBatchGroupCells);
   std::vector<int> group(ninst);
   long long before = 0;
   for (int i : order) {  // by the middle of the instance's cells
@@ -1511,8 +1554,12 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
     before += n;
   }
   b->groups.resize((size_t)ngroup);
-  for (int i : order)
-    b->groups[group[i]].maxsteps = std::max(b->groups[group[i]].maxsteps, b->inst[i].nsteps);
+  for (int i : order) {
+    const hs2::BatchInst &I = b->inst[i];
+    batch_group &g = b->groups[group[i]];
+    g.maxsteps = std::max(g.maxsteps, I.nsteps);
+    g.work += (long long)I.nz * I.ny * I.nx * I.nsteps;
+  }
   for (int k = 0; k < NKIND && rc == HS2_OK; k++) {
     std::vector<int> b0(ninst, 0), owner;
     for (int i : order) {
@@ -1532,7 +1579,18 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
                     hipMemcpyHostToDevice), "hipMemcpy");
     }
   }
-  if (rc == HS2_OK) bad(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "stream");
+  // the longest group first, each to the lane with the least work so far
+  std::sort(b->groups.begin(), b->groups.end(),
+            [](const batch_group &x, const batch_group &y) { return x.work > y.work; });
+  long long load[kBatchLanes] = {};
+  for (batch_group &g : b->groups) {
+    g.lane = (int)(std::min_element(load, load + kBatchLanes) - load);
+    load[g.lane] += g.work;
+  }
+  for (int lane = 0; lane < kBatchLanes; lane++)
+    if (rc == HS2_OK && (lane == 0 || load[lane] > 0))
+      bad(hipStreamCreateWithFlags(&b->stream[lane], hipStreamNonBlocking), "stream");
+  if (rc == HS2_OK) bad(hipEventCreateWithFlags(&b->ev_lane, hipEventDisableTiming), "event");
   if (rc == HS2_OK) bad(hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming), "event");
   if (rc == HS2_OK) bad(hipEventCreateWithFlags(&b->ev_out, hipEventDisableTiming), "event");
   if (rc != HS2_OK) {
@@ -1602,22 +1660,23 @@ int hs2_batch_forward(hs2_batch *b, double *d_T, const double *d_src, double *d_
     return fail(HS2_E_ARG, "hs2_batch_forward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
   HIP_TRY(hipEventRecord(b->ev_in, (hipStream_t)stream));
-  HIP_TRY(hipStreamWaitEvent(b->stream, b->ev_in, 0));
-  for (batch_group &g : b->groups) {
-    if (!g.maxsteps) continue;
-    HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 0, 0, 0, b->stream));
-    const int C = std::min(b->chunk, g.maxsteps);
-    const int reps = (g.maxsteps + C - 1) / C;
-    const std::vector<const void *> key = {d_T, d_src, d_hist, d_work, b->dv.M, b->dv.w,
-                                           b->dv.g[0], b->dv.g[1], b->dv.g[2],
-                                           (const void *)(intptr_t)C};
-    const int rc = batch_replay(
-        b, &g.fwd_exec, &g.fwd_key, key, reps,
-        [&](hipStream_t s) { return emit_forward(b, g, d_T, d_src, d_hist, w, C, s); },
-        "hs2_batch_forward");
-    if (rc != HS2_OK) return rc;
-  }
-  HIP_TRY(hipEventRecord(b->ev_out, b->stream));
+  HIP_TRY(hipStreamWaitEvent(b->stream[0], b->ev_in, 0));
+  HIP_TRY(hipEventRecord(b->ev_lane, b->stream[0]));
+  auto chunk = [&](const batch_group &g) { return std::min(b->chunk, g.maxsteps); };
+  const int rc = batch_lanes(
+      b, 0, [&](const batch_group &g) { return (g.maxsteps + chunk(g) - 1) / chunk(g); },
+      [&](batch_group &g, hipStream_t st) {
+        const int C = chunk(g);
+        const std::vector<const void *> key = {d_T, d_src, d_hist, d_work, b->dv.M, b->dv.w,
+                                               b->dv.g[0], b->dv.g[1], b->dv.g[2],
+                                               (const void *)(intptr_t)C};
+        return batch_replay(
+            b, st, &g.fwd_exec, &g.fwd_key, key,
+            [&](hipStream_t s) { return emit_forward(b, g, d_T, d_src, d_hist, w, C, s); },
+            "hs2_batch_forward");
+      });
+  if (rc != HS2_OK) return rc;
+  HIP_TRY(hipEventRecord(b->ev_out, b->stream[0]));
   HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
   return HS2_OK;
 }
@@ -1631,7 +1690,7 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   if (work_doubles < (size_t)batch_work_doubles(b))
     return fail(HS2_E_ARG, "hs2_batch_backward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
-  hipStream_t s = b->stream;
+  hipStream_t s = b->stream[0];
   HIP_TRY(hipEventRecord(b->ev_in, (hipStream_t)stream));
   HIP_TRY(hipStreamWaitEvent(s, b->ev_in, 0));
   HIP_TRY(hs2::launch_fill(d_gM, b->N, 0.0, s));
@@ -1642,19 +1701,19 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   const std::vector<const void *> key = {d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc,
                                          d_work, b->dv.M, b->dv.w, b->dv.g[0], b->dv.g[1],
                                          b->dv.g[2]};
-  for (batch_group &g : b->groups) {
-    if (!g.maxsteps) continue;
-    HIP_TRY(hs2::launch_batch_counter(b->d_ctr, 1, 0, 0, s));
-    const int reps = (g.maxsteps + b->K - 1) / b->K;
-    const int rc = batch_replay(
-        b, &g.bwd_exec, &g.bwd_key, key, reps,
-        [&](hipStream_t st) {
-          return emit_backward_segment(b, g, d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc, w,
-                                       st);
-        },
-        "hs2_batch_backward");
-    if (rc != HS2_OK) return rc;
-  }
+  HIP_TRY(hipEventRecord(b->ev_lane, s));
+  const int rc = batch_lanes(
+      b, 1, [&](const batch_group &g) { return (g.maxsteps + b->K - 1) / b->K; },
+      [&](batch_group &g, hipStream_t st) {
+        return batch_replay(
+            b, st, &g.bwd_exec, &g.bwd_key, key,
+            [&](hipStream_t s) {
+              return emit_backward_segment(b, g, d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx,
+                                           d_gsrc, w, s);
+            },
+            "hs2_batch_backward");
+      });
+  if (rc != HS2_OK) return rc;
   HIP_TRY(hipEventRecord(b->ev_out, s));
   HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
   return HS2_OK;

@@ -1,6 +1,6 @@
 // Batched execution of many independent ADI problems of different sizes and
-// step counts: one launch per sweep covers every instance of a group (the
-// groups run one after another; see kBatchGroupCells).  Each launch kind
+// step counts: one launch per sweep covers every instance of a group (groups
+// run two at a time; see kBatchGroupCells).  Each launch kind
 // has a block -> instance table; a block finds its instance, its local block
 // index and its instance's current step, and works on that instance's slice
 // of the concatenated fields (per-voxel coefficients, DenseView).
@@ -26,14 +26,17 @@ constexpr int kBatchWaves = 4;     // waves (units of rows) per block of the x k
 constexpr int kBatchSeg = 8;       // cells per thread segment of the line kernels
 constexpr int kBatchPlanes = 2;    // planes a wave of the x sweep walks (1, 4: 2% slower, 8: 18%)
 constexpr int kBatchSensPlanes = 8;  // planes per block of the sensitivity pass
-// Cells of a group, about: a step's fields (T, T*, M, three conductances, w: 49
-// bytes a cell) then fit the 256 MB Infinity Cache, and launches stay long.
-// ns per cell and step by the cells run together, forward | with gradient:
-// 12.7 million 0.0265 | 0.1023, 8.7 0.0259 | 0.1013, 4.2 to 4.8 0.0241 | 0.0953,
-// 3.3 0.0261, 2.6 0.1029, 2.0 0.0305.  24 instances of 32..128^3 and 40 to 160
-// steps: histories 29.7 -> 28.0 ms (0.6 of it one counter launch a chunk instead
-// of one a step), gradients 118.1 -> 113.1.
-constexpr long long kBatchGroupCells = 4500000;
+// Cells of a group, about: two groups run side by side (kBatchLanes), and a
+// step's fields of both (T, T*, M, three conductances, w: 49 bytes a cell) fit the
+// 256 MB Infinity Cache.  ns per cell and step by the cells run together on one
+// stream, forward | with gradient: 12.7 million 0.0265 | 0.1023, 8.7 0.0259 |
+// 0.1013, 4.2 to 4.8 0.0241 | 0.0953, 2.0 to 2.6 0.0305 | 0.1029.  24 instances of
+// 32..128^3 and 40 to 160 steps, ms for histories | gradients: all together 29.7 |
+// 118.1, groups of 4.5 million one by one 28.0 | 113.1, on two lanes of 4.5 million
+// 26.6 | 109.7, of 3 million 25.4 | 106.9, of 2.25 million 24.9 | 107.4, of 1.5
+// million 26.6 | 110.6; three lanes of 1.5 million 25.3 | 108.5, four of 1.2 31.4 |
+// 116.7.
+constexpr long long kBatchGroupCells = 2250000;
 constexpr int kBatchAlign = 32;    // instance offsets are multiples of this many cells
 
 // Segments of kBatchSeg cells per line of L cells in the y and z line

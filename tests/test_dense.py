@@ -137,14 +137,14 @@ def test_gradients_do_not_depend_on_the_workspace(every):
 
 
 EDGES = [s for s in SHAPES if max(s) <= 128] + [(2, 1, 31), (5, 127, 127), (128, 9, 34)]
-# two groups of instances that run one after the other, a small one in each
+# three groups of instances on two streams
 GROUPS = [(128, 128, 128), (7, 9, 33), (127, 128, 120), (128, 125, 128), (40, 3, 17)]
 
 
 @pytest.mark.parametrize("shapes", [EDGES, GROUPS], ids=["edges", "groups"])
 def test_batches_match_single_plans(shapes):
     """Every row shape of the batched kernels and cut and whole columns in one
-    batch, and a batch that is worked off in two groups; unequal step counts, a
+    batch, and a batch that is worked off in three groups; unequal step counts, a
     source in some: each instance against a plan of its own (other shapes, the
     same algebra: 1e-12 of the largest value)."""
     steps = [2 + (3 * i) % 7 for i in range(len(shapes))]
