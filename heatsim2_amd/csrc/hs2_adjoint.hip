@@ -286,7 +286,8 @@ hipError_t launch_adj_line(const Grid &g, const ClassView &v, int axis, const do
 }
 hipError_t launch_adj_line(const Grid &g, const DenseView &v, int axis, const double *R,
                            int scale_m, double *U, hipStream_t s) {
-  if (axis == 2 ? dense_rows_ok(g) : dense_cols_ok(g, axis))
+  // (z lines that hs2_dense.hip serves are solved with lambda, launch_dense_lambda)
+  if (axis == 2 ? dense_rows_ok(g) : axis == 1 && dense_cols_ok(g, 1))
     return launch_dense_adj(g, v, axis, R, scale_m, U, s);
   return launch_adj_line_v(g, v, axis, R, scale_m, U, s);
 }

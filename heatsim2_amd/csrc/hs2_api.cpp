@@ -90,7 +90,7 @@ struct hs2_plan {
   hs2::SConfig scfg[2] = {{0, 0}, {0, 0}};  // [0] z, [1] y
 };
 
-enum { KIND_X2 = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, KIND_SENS = 5, NKIND = 6 };
+enum { KIND_X = 0, KIND_Y = 1, KIND_Z = 2, KIND_AX = 3, KIND_CELL = 4, KIND_SENS = 5, NKIND = 6 };
 
 // Instances that run together: a range of blocks of every launch kind.  The
 // groups of a lane run one after another on the lane's stream, on its two
@@ -220,7 +220,7 @@ hs2::Grid grid_of(const hs2_plan *p) { return hs2::Grid{p->grid.nz, p->grid.ny, 
 hipError_t sweep_x(const hs2_plan *p, const double *Tn, double *Ts, const uint8_t *vmap,
                    const double *vtab, const double *sfield, hipStream_t s, bool ry = false) {
   const hs2::Grid g = grid_of(p);
-  if (p->use_lines && p->rows.g) 
+  if (p->use_lines && p->rows.g)
     return hs2::launch_rows(g, p->rows, Tn, Ts, vmap, vtab, sfield, ry, s);
   if (p->mode == MODE_CLASS && p->have_comb && p->use_comb && !vmap && !sfield &&
       hs2::x_ry_ok(p->xcfg, g))
@@ -380,7 +380,7 @@ hs2::BatchMap batch_map(const hs2_batch *b, const batch_group &g, int kind, int 
 
 int blocks_of(const hs2::BatchInst &I, int kind) {
   switch (kind) {
-    case KIND_X2: return (I.units + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
+    case KIND_X: return (I.units + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
     case KIND_Y: return (I.nx * I.nz + I.cw[1] - 1) / I.cw[1];
     case KIND_Z: return (I.nx * I.ny + I.cw[0] - 1) / I.cw[0];
     case KIND_AX: return (I.rows + hs2::kBatchWaves - 1) / hs2::kBatchWaves;
@@ -429,18 +429,18 @@ BatchWork batch_work(const hs2_batch *b, double *w) {
 }
 
 // forward: `steps` steps (ckpt store, x, y, z with the readout, tick)
-hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const double *src, double *hist,
-                        const BatchWork &w, int steps, hipStream_t s) {
+hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const double *src,
+                        double *hist, const BatchWork &w, int steps, hipStream_t s) {
   hipError_t e = hipSuccess;
   for (int c = 0; c < steps && e == hipSuccess; c++) {
-    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X2, hs2::RULE_FWD, c), g.nblk[KIND_X2], b->dv,
-                               T, w.ws, src, w.ck, true, s);
+    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X, hs2::RULE_FWD, c), g.nblk[KIND_X],
+                               b->dv, T, w.ws, src, w.ck, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Y, hs2::RULE_FWD, c), g.nblk[KIND_Y], 1, b->dv,
-                                 T, w.ws, w.ws, nullptr, true, s);
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Y, hs2::RULE_FWD, c), g.nblk[KIND_Y], 1,
+                                 b->dv, T, w.ws, w.ws, nullptr, true, s);
     if (e == hipSuccess)
-      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Z, hs2::RULE_FWD, c), g.nblk[KIND_Z], 0, b->dv,
-                                 T, w.ws, T, hist, false, s);
+      e = hs2::launch_batch_cols(batch_map(b, g, KIND_Z, hs2::RULE_FWD, c), g.nblk[KIND_Z], 0,
+                                 b->dv, T, w.ws, T, hist, false, s);
   }
   if (e == hipSuccess) e = hs2::launch_batch_counter(b->d_ctr + 2 * g.lane, 0, steps, 1, s);
   return e;
@@ -448,7 +448,8 @@ hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const dou
 
 // one backward segment: load checkpoints, recompute its K steps keeping every
 // state, K adjoint steps, tick
-hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const double *src, const double *ghist,
+hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const double *src,
+                                 const double *ghist,
                                  double *gM, double *gz, double *gy, double *gx, double *gsrc,
                                  const BatchWork &w, hipStream_t s) {
   const int K = b->K;
@@ -458,8 +459,8 @@ hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const doubl
   for (int j = 0; j < K && e == hipSuccess; j++) {
     const double *in = w.seg + (size_t)j * N;
     double *tx = w.segx + (size_t)j * N, *ty = w.segy + (size_t)j * N;
-    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X2, hs2::RULE_RECOMP, j), g.nblk[KIND_X2], b->dv,
-                               in, tx, src, nullptr, false, s);
+    e = hs2::launch_batch_rows(batch_map(b, g, KIND_X, hs2::RULE_RECOMP, j), g.nblk[KIND_X],
+                               b->dv, in, tx, src, nullptr, false, s);
     if (e == hipSuccess)
       e = hs2::launch_batch_cols(batch_map(b, g, KIND_Y, hs2::RULE_RECOMP, j), g.nblk[KIND_Y], 1,
                                  b->dv, in, tx, ty, nullptr, false, s);

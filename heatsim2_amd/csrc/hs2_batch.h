@@ -139,6 +139,7 @@ hipError_t launch_batch_rows(const BatchMap &m, int nblocks, const DenseView &v,
 hipError_t launch_batch_cols(const BatchMap &m, int nblocks, int axis, const DenseView &v,
                              const double *Tn, const double *Y, double *X, double *hist, bool ry,
                              hipStream_t s);
+// transposed y or x solves (axis 1, 2)
 hipError_t launch_batch_adj_line(const BatchMap &m, int nblocks, int axis, const DenseView &v,
                                  const double *R, int scale_m, double *U, hipStream_t s);
 hipError_t launch_batch_lambda(const BatchMap &m, int nblocks, const DenseView &v, const double *u,

@@ -11,11 +11,12 @@
 // us, the kernels before (rows staged through LDS, both end rows of every
 // segment reduced) | now:
 //                      64x128x128      48x96x120 (per side)   24 of 32..128^3
+//                                                             (in one launch)
 //   x                  13.1 | 10.4     13.3 | 9.5             121 | 73
 //   y after x / alone  10.5 | 7.3/8.4   9.3 | 7.5              68 | 49/64
 //   z                   9.3 | 9.3      10.3 | 7.4              61 | 58
 //   transposed x        16.5 | 6.8      -                      74 | 41
-//   transposed y / z    10.8 | 8.5, 11.8 | 7.9                 59 | 52, 56 | 50
+//   transposed y        10.8 | 8.5      -                      59 | 52
 // 10.4 us for 51 MB is 4.9 TB/s, what a copy between arrays larger than the
 // Infinity Cache reaches; 29x45x51 (3.5 to 5.2 us a launch) is bound by the
 // latency of one chain of load, solve and store.
@@ -271,15 +272,16 @@ __device__ __forceinline__ void col_sweep(const Grid &g, const V &v, int P, int 
   if (AXIS == 0 && surf && c.p == 0 && c.L >= 2) surf[c.base] = surface_readout(xs, x1, dz);
 }
 
-// Transposed y and z solves: A_a^T U = (scale_m ? M R : R).  U must not alias R.
-template <class V, int SEG, int AXIS>
+// Transposed y solve: A_y^T U = (scale_m ? M R : R).  U must not alias R.  (z's is
+// col_lambda's.)
+template <class V, int SEG>
 __device__ __forceinline__ void col_adjoint(const Grid &g, const V &v, int P, int CW,
                                             const double *R, int scale_m, double *U, int blk) {
   extern __shared__ double lds[];
-  const ColPlace c = col_place<AXIS>(g, SEG, P, CW, blk);
+  const ColPlace c = col_place<1>(g, SEG, P, CW, blk);
   const unsigned n = (unsigned)g.nx * (unsigned)g.ny * (unsigned)g.nz;
   const BufRsrc bR = make_buf(R, n * 8u), bU = make_buf(U, n * 8u), bM = make_buf(v.M, n * 8u),
-                bG = make_buf(v.g[AXIS], n * 8u), bW = make_buf(v.w, n);
+                bG = make_buf(v.g[1], n * 8u), bW = make_buf(v.w, n);
   const unsigned so = c.so * 8u, vo = c.vo * 8u;
   double r[SEG], M[SEG], G[SEG + 1];
   uint32_t w[SEG + 2];
@@ -537,10 +539,10 @@ __global__ __launch_bounds__(256) void k_drows_adj(Grid g, V v, const double *R,
   if (unit < units) row_adjoint<V, CPL, G>(g, v, R, scale_m, U, unit);
 }
 
-template <class V, int SEG, int AXIS>
+template <class V, int SEG>
 __global__ __launch_bounds__(512) void k_dcols_adj(Grid g, V v, int P, int CW, const double *R,
                                                    int scale_m, double *U) {
-  col_adjoint<V, SEG, AXIS>(g, v, P, CW, R, scale_m, U,
+  col_adjoint<V, SEG>(g, v, P, CW, R, scale_m, U,
                             xcd_remap_chunks<32>(blockIdx.x, gridDim.x));
 }
 
@@ -637,8 +639,8 @@ static hipError_t launch_dcols_t(const Grid &g, const V &v, int axis, int P, int
   const dim3 grid((unsigned)((ncol + CW - 1) / CW)), block(P * CW);
   const size_t shm = sizeof(double) * 6 * P * CW;
 #define HS2_RUN(AXIS, RY)                                                                        \
-  hipLaunchKernelGGL((k_dcols<V, SEG, AXIS, RY>), grid, block, shm, s, g, v, P, CW, Tn, Y, X, surf, \
-                     dz)
+  hipLaunchKernelGGL((k_dcols<V, SEG, AXIS, RY>), grid, block, shm, s, g, v, P, CW, Tn, Y, X,    \
+                     surf, dz)
   if (axis == 1 && ry) HS2_RUN(1, true);
   else if (axis == 1) HS2_RUN(1, false);
   else if (!ry) HS2_RUN(0, false);
@@ -697,16 +699,15 @@ hipError_t launch_dense_adj(const Grid &g, const DenseView &v, int axis, const d
     return hipGetLastError();
   }
   int seg, P, CW;
-  const long long ncol = (long long)g.nx * (axis == 1 ? g.nz : g.ny);
-  dcol_shape(axis == 1 ? g.ny : g.nz, ncol, &seg, &P, &CW);
+  const long long ncol = (long long)g.nx * g.nz;
+  dcol_shape(g.ny, ncol, &seg, &P, &CW);
   const dim3 grid((unsigned)((ncol + CW - 1) / CW)), block(P * CW);
   const size_t shm = sizeof(double) * 6 * P * CW;
-#define HS2_RUN(SEG, AXIS)                                                                       \
-  if (seg == SEG && axis == AXIS)                                                                \
-    hipLaunchKernelGGL((k_dcols_adj<DenseView, SEG, AXIS>), grid, block, shm, s, g, v, P, CW, R, \
-                       scale_m, U);
-  HS2_RUN(8, 0) HS2_RUN(16, 0) HS2_RUN(8, 1) HS2_RUN(16, 1)
-#undef HS2_RUN
+  if (seg == 8)
+    hipLaunchKernelGGL((k_dcols_adj<DenseView, 8>), grid, block, shm, s, g, v, P, CW, R, scale_m, U);
+  else
+    hipLaunchKernelGGL((k_dcols_adj<DenseView, 16>), grid, block, shm, s, g, v, P, CW, R, scale_m,
+                       U);
   return hipGetLastError();
 }
 
@@ -740,8 +741,9 @@ hipError_t launch_dense_sens(const Grid &g, const DenseView &v, const AdjGroup &
 // One launch covers every instance (axis lengths <= kBatchMaxLen); see
 // hs2_batch.h for the block mapping.
 template <bool RY>
-__global__ __launch_bounds__(kBatchWaves *kWave) void kb_rows(BatchMap m, DenseView v, const double *Tn,
-                                               double *Ts, const double *src, double *ck) {
+__global__ __launch_bounds__(kBatchWaves *kWave) void kb_rows(BatchMap m, DenseView v,
+                                                              const double *Tn, double *Ts,
+                                                              const double *src, double *ck) {
   BatchInst I;
   int local, t;
   if (!batch_locate(m, I, local, t)) return;
@@ -780,8 +782,9 @@ __global__ __launch_bounds__(kBatchThreads) void kb_cols(BatchMap m, DenseView v
       I.cw[AXIS], Tn + I.off, Y + I.off, X + I.off, surf, I.dz, local);
 }
 
-__global__ __launch_bounds__(kBatchWaves *kWave) void kb_rows_adj(BatchMap m, DenseView v, const double *R,
-                                                   int scale_m, double *U) {
+__global__ __launch_bounds__(kBatchWaves *kWave) void kb_rows_adj(BatchMap m, DenseView v,
+                                                                  const double *R, int scale_m,
+                                                                  double *U) {
   BatchInst I;
   int local, t;
   if (!batch_locate(m, I, local, t)) return;
@@ -799,16 +802,15 @@ __global__ __launch_bounds__(kBatchWaves *kWave) void kb_rows_adj(BatchMap m, De
 #undef HS2_ROW
 }
 
-template <int AXIS>
 __global__ __launch_bounds__(kBatchThreads) void kb_cols_adj(BatchMap m, DenseView v,
                                                              const double *R, int scale_m,
                                                              double *U) {
   BatchInst I;
   int local, t;
   if (!batch_locate(m, I, local, t)) return;
-  col_adjoint<DenseView, kBatchSeg, AXIS>(
-      Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off), batch_line_segs(AXIS == 1 ? I.ny : I.nz),
-      I.cw[AXIS], R + I.off, scale_m, U + I.off, local);
+  col_adjoint<DenseView, kBatchSeg>(Grid{I.nz, I.ny, I.nx}, offset_view(v, I.off),
+                                    batch_line_segs(I.ny), I.cw[1], R + I.off, scale_m,
+                                    U + I.off, local);
 }
 
 // u: the previous step's solves (uz, uy, ux, N apart); in the last step of an
@@ -885,13 +887,12 @@ hipError_t launch_batch_cols(const BatchMap &m, int nblocks, int axis, const Den
 
 hipError_t launch_batch_adj_line(const BatchMap &m, int nblocks, int axis, const DenseView &v,
                                  const double *R, int scale_m, double *U, hipStream_t s) {
-  const size_t shm = sizeof(double) * 6 * (size_t)kBatchThreads;
-  const dim3 grid(nblocks), block(kBatchThreads);
-  switch (axis) {
-    case 0: hipLaunchKernelGGL(kb_cols_adj<0>, grid, block, shm, s, m, v, R, scale_m, U); break;
-    case 1: hipLaunchKernelGGL(kb_cols_adj<1>, grid, block, shm, s, m, v, R, scale_m, U); break;
-    default: hipLaunchKernelGGL(kb_rows_adj, grid, dim3(kBatchWaves * kWave), 0, s, m, v, R, scale_m, U); break;
-  }
+  if (axis == 1)
+    hipLaunchKernelGGL(kb_cols_adj, dim3(nblocks), dim3(kBatchThreads),
+                       sizeof(double) * 6 * (size_t)kBatchThreads, s, m, v, R, scale_m, U);
+  else
+    hipLaunchKernelGGL(kb_rows_adj, dim3(nblocks), dim3(kBatchWaves * kWave), 0, s, m, v, R,
+                       scale_m, U);
   return hipGetLastError();
 }
 

@@ -67,7 +67,7 @@ hipError_t launch_dense_cols(const Grid &g, const DenseView &v, int axis, const 
 hipError_t launch_dense_cols(const Grid &g, const AsymView &v, int axis, const double *Tn,
                              const double *Y, double *X, double *surf, double dz, bool ry,
                              hipStream_t s);
-// U = A_axis^{-T} (scale_m ? M R : R) along every line of `axis`
+// U = A_axis^{-T} (scale_m ? M R : R) along every line of `axis` (x or y)
 hipError_t launch_dense_adj(const Grid &g, const DenseView &v, int axis, const double *R,
                             int scale_m, double *U, hipStream_t s);
 
