@@ -285,13 +285,16 @@ __device__ __forceinline__ double scan_down(double v, const double *b, unsigned 
 // right-hand side is staged and no class byte is read.  Bound by the row
 // loads through L1 and L2 at large sizes (256^3: 56 us, 4.8 TB/s of 16 B per
 // cell, against 72 for the staged class kernel; 128 x 512 x 512: 145 us
-// against 198), by latency at small ones (61 x 149 x 203: 12.5 against 25
-// us, 40^3: 3.9 against 5.6).  The factors are read from LDS for every row: in
+// against 198), by latency at small ones (61 x 149 x 203: 12.1 against 25
+// us, 40^3: 3.8 against 5.6).  The factors are read from LDS for every row: in
 // registers they cost a wave per SIMD (61 us at 256^3).  Lanes of more than 6
 // cells do worse than two waves per row (512 cells: 178 us against 145): their
 // loads are 64 bytes apart, and too few waves fit; rows put in lane order
 // through LDS made whole-line loads and stores of it (170 us there, but 60 at
-// 256^3).
+// 256^3).  Waves in flight weigh most: two rows to a wave (a third of the row
+// loads saved, 160 registers) take 69 us at 256^3 and 170 at 512 cells; the next
+// plane's rows loaded during the solve 55 and 151; five waves per SIMD in 96
+// registers 58 and 156.
 template <int CPL, int G, int W, bool SRC, bool RY>
 __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__restrict__ Tn,
                                               double *__restrict__ Ts,
