@@ -21,7 +21,8 @@ int default_strided(int L, SConfig *cfg);
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 // ry: the x sweep writes y's right-hand side M T* - (Ly/2) T^n instead of T*
 // and the y sweep reads it (class maps, steps without sources, x shapes for
-// which x_ry_ok holds); the z sweep is unchanged
+// which x_ry_ok holds; per-voxel coefficients where dense_ry holds); the z sweep
+// is unchanged
 bool x_ry_ok(XConfig c, const Grid &g);
 
 hipError_t launch_sweep_x(XConfig cfg, const Grid &g, const ClassView &v, const double *Tn,

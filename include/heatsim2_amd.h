@@ -112,17 +112,20 @@ int hs2_plan_expand(hs2_plan *plan, double *d_M, double *d_w, double *d_gz, doub
  * block's lines one after the other in (z, y) order; a proper divisor of
  * x_lines tiles them as x_lines/x_lines_y planes x x_lines_y rows, which
  * share more neighbour rows.  y and z sweeps: segments of *_seg cells per
- * thread, *_lines lines per block (segments*lines <= 512).  No upstream
- * counterpart. */
+ * thread, *_lines lines per block (segments*lines <= 512).  On per-voxel
+ * coefficients x rows of up to 256 cells and y and z lines of up to 512 have
+ * shapes of their own; a configuration is checked and kept there, but not
+ * used.  No upstream counterpart. */
 int hs2_plan_set_config(hs2_plan *plan, int x_cpl, int x_lanes, int x_lines, int x_lines_y,
                         int y_seg, int y_lines, int z_seg, int z_lines);
 
 /* Plan options (no upstream counterpart).
  *   HS2_OPT_COMBINED_X (default 1): with class maps, let the x sweep of
  *     source-free steps read one combined class byte per cell (the id of
- *     the cell's z, y, x class triple, built by hs2_plan_set_compact when
- *     there are 256 triples or fewer) instead of the three class planes;
- *     0 reads the three planes.  Same numbers either way.
+ *     the cell's z, y, x class triple, when there are 256 triples or fewer;
+ *     built for plans without line tables for x and when they are switched
+ *     off) instead of the three class planes; 0 reads the three planes.
+ *     Same numbers either way.
  *   HS2_OPT_LINE_TABLES (default 1; hs2_plan_set_config sets it to 0, since
  *     its shapes are the other kernels'): with class maps, sweep the axes
  *     whose lines fall into few distinct ones with those lines' factors,
@@ -141,7 +144,7 @@ int hs2_plan_get_option(const hs2_plan *plan, int option, int *value);
  * right-hand side M T* - (Ly/2) T^n from the x sweep (16 B per cell less field
  * traffic per step than writing T* and re-reading T^n) else 0, and the
  * number of combined class ids the x sweep of source-free steps reads (0:
- * it reads the three class planes). */
+ * it reads the three class planes, or line tables). */
 int hs2_plan_info(const hs2_plan *plan, int *info);
 
 /* One full Douglas step T^n -> T^{n+1} (x, y, z substeps).
@@ -229,10 +232,11 @@ int hs2_grad_backward(hs2_plan *plan, int nsteps, int ckpt_every, const double *
 
 /* ---- Batches (no upstream counterpart).  Many independent problems of
  * different sizes and step counts, each with per-voxel coefficients, run
- * forward and adjoint together: one launch per sweep covers every
- * instance, and the time loop is a captured HIP graph (a chunk of forward
- * steps, or one checkpoint segment of the backward pass) replayed on an
- * internal stream ordered after `stream`.  Axis lengths 1..128 (nz >= 2).
+ * forward and adjoint together, in groups of about 2.25 million cells, two
+ * groups side by side: one launch per sweep covers a group, and its time loop
+ * is a captured HIP graph (a chunk of forward steps, or one checkpoint segment
+ * of the backward pass) replayed on an internal stream ordered after
+ * `stream`.  Axis lengths 1..128 (nz >= 2).
  * All fields are the instances' fields concatenated at the offsets that
  * hs2_batch_layout reports (16-byte aligned; padding cells are ignored). */
 typedef struct hs2_batch hs2_batch;
