@@ -38,7 +38,7 @@ EXPORTS = ("hs2_plan_create", "hs2_plan_destroy", "hs2_plan_set_compact", "hs2_p
            "hs2_plan_set_dense_asym", "hs2_plan_expand", "hs2_plan_set_config", "hs2_plan_set_option",
            "hs2_plan_get_option", "hs2_plan_info",
            "hs2_step", "hs2_run",
-           "hs2_run_timed", "hs2_grad_work_doubles", "hs2_grad_forward", "hs2_grad_backward",
+           "hs2_run_timed", "hs2_grad_work_doubles", "hs2_grad_work_best", "hs2_grad_forward", "hs2_grad_backward",
            "hs2_batch_create", "hs2_batch_destroy", "hs2_batch_layout", "hs2_batch_set_dense",
            "hs2_batch_set_options", "hs2_batch_forward", "hs2_batch_backward",
            "hs2_step_noalloc", "hs2_surface_temperature", "hs2_last_error", "hs2_version")
@@ -84,6 +84,8 @@ def load():
     L.hs2_run_timed.restype = i32
     L.hs2_grad_work_doubles.argtypes = [vp, i32]
     L.hs2_grad_work_doubles.restype = ctypes.c_size_t
+    L.hs2_grad_work_best.argtypes = [vp, i32, i32]
+    L.hs2_grad_work_best.restype = ctypes.c_size_t
     L.hs2_grad_forward.argtypes = [vp, vp, i32, i32, vp, vp, vp, i32, vp, vp]
     L.hs2_grad_forward.restype = i32
     L.hs2_grad_backward.argtypes = [vp, i32, i32, vp, vp, vp, i32, vp, vp, vp, vp, vp, vp, vp, vp,

@@ -157,6 +157,20 @@ class GradPlan(object):
             self.plan = None
 
 
+def _workspace(gplan, nsteps, ckpt_every, dev):
+    """hs2_grad_backward's scratch: the fastest size that the device has memory
+    for, down to the least (the same bits with each)."""
+    L = _lib.load()
+    least = int(L.hs2_grad_work_doubles(gplan.plan, ckpt_every))
+    best = int(L.hs2_grad_work_best(gplan.plan, nsteps, ckpt_every))
+    for size in sorted({best, min(best, least + 7 * gplan.n)}, reverse=True):
+        try:
+            return torch.empty(size, dtype=torch.float64, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return torch.empty(least, dtype=torch.float64, device=dev)
+
+
 class _SurfaceHistory(torch.autograd.Function):
     @staticmethod
     def forward(ctx, gplan, nsteps, ckpt_every, src_steps, w, M, gz, gy, gx, T0, *src):
@@ -188,18 +202,17 @@ class _SurfaceHistory(torch.autograd.Function):
             ctx.coef = gplan._coef
         ghist = ghist.to(dev, torch.float64).contiguous()
         shape = gplan.shape
-        work_n = int(L.hs2_grad_work_doubles(gplan.plan, ctx.ckpt_every))
-        work = torch.empty(work_n, dtype=torch.float64, device=dev)
         gM, gz, gy, gx, gT0 = (torch.empty(shape, dtype=torch.float64, device=dev)
                                for _ in range(5))
         nsrc = len(ctx.src_steps)
         gsrc = torch.empty((nsrc,) + shape, dtype=torch.float64, device=dev) if nsrc else None
+        work = _workspace(gplan, ctx.nsteps, ctx.ckpt_every, dev)  # last: it takes what is left
         steps = (ctypes.c_int32 * max(nsrc, 1))(*ctx.src_steps)
         _lib.check("hs2_grad_backward", L.hs2_grad_backward(
             gplan.plan, ctx.nsteps, ctx.ckpt_every, _lib.ptr(ctx.ckpt), _lib.ptr(ctx.srcs),
             steps if nsrc else None, nsrc, _lib.ptr(ghist), _lib.ptr(gM), _lib.ptr(gz),
             _lib.ptr(gy), _lib.ptr(gx), _lib.ptr(gsrc), _lib.ptr(gT0), _lib.ptr(work),
-            ctypes.c_size_t(work_n), _lib.stream_handle()))
+            ctypes.c_size_t(work.numel()), _lib.stream_handle()))
         gsrcs = tuple(gsrc[i] for i in range(nsrc)) if nsrc else ()
         return (None, None, None, None, None, gM, gz, gy, gx, gT0) + gsrcs
 
@@ -212,7 +225,9 @@ def surface_history(gplan, coef, T0, nsteps, sources=(), ckpt_every=50):
     sequence of (step, field) with field the volumetric power density
     (W/m^3) added during that step (at most one per step); ckpt_every:
     steps between checkpoints (memory: ceil(nsteps/ckpt_every) +
-    3*ckpt_every + 6 fields).  Gradients flow to M, g, T0 and the source fields.
+    3*ckpt_every + 13 fields, on grids of up to 4 million cells and several
+    segments another 3*ckpt_every + 1; 3*ckpt_every + 6 where the device has no
+    more).  Gradients flow to M, g, T0 and the source fields.
     """
     nsteps, ckpt_every = int(nsteps), int(ckpt_every)
     if nsteps < 1 or ckpt_every < 1:

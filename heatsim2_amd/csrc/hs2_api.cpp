@@ -297,6 +297,10 @@ bool grad_grouped(const hs2_plan *p) {
 // 75.6 | 68.6, 100x128x160 156 | 146, 128x160x160 231 | 221, 160x200x200 481 |
 // 469: beyond, 2% is not worth a second store of states.
 constexpr size_t kOverlapCells = 4000000;
+// the most bytes that second store is asked for: 50 steps a segment at four
+// million cells take 4.8 GB; segments of many hundred steps are not worth twice
+// their memory
+constexpr size_t kMostSecondStore = size_t(8) << 30;
 bool grad_overlaps(const hs2_plan *p) { return grad_grouped(p) && (size_t)p->n <= kOverlapCells; }
 
 // the second stream is there and `s` is not being captured
@@ -1328,9 +1332,17 @@ int hs2_run_timed(hs2_plan *p, double *d_T, int nsteps, int method, double *kern
 
 size_t hs2_grad_work_doubles(const hs2_plan *p, int ckpt_every) {
   if (!p || ckpt_every < 1) return 0;
-  const size_t K = (size_t)ckpt_every, n = (size_t)p->n;
-  if (!grad_grouped(p)) return (3 * K + 6) * n;
-  return ((grad_overlaps(p) ? 2 : 1) * (3 * K + 1) + 3 * hs2::kAdjGroup) * n;
+  return (3 * (size_t)ckpt_every + 6) * (size_t)p->n;
+}
+
+size_t hs2_grad_work_best(const hs2_plan *p, int nsteps, int ckpt_every) {
+  if (!p || nsteps < 1 || ckpt_every < 1) return 0;
+  const size_t n = (size_t)p->n, store = (3 * (size_t)ckpt_every + 1) * n;
+  if (!grad_grouped(p)) return hs2_grad_work_doubles(p, ckpt_every);
+  // a second store only where there is a second segment to recompute into it
+  const bool two = grad_overlaps(p) && nsteps > ckpt_every &&
+                   store <= kMostSecondStore / sizeof(double);
+  return (two ? 2 : 1) * store + 3 * hs2::kAdjGroup * n;
 }
 
 int hs2_grad_forward(hs2_plan *p, double *d_T, int nsteps, int ckpt_every, double *d_ckpt,
@@ -1374,7 +1386,7 @@ int hs2_grad_backward(hs2_plan *p, int nsteps, int ckpt_every, const double *d_c
   if (p->grid.nz < 2) return fail(HS2_E_ARG, "hs2_grad_backward: the surface readout needs nz >= 2");
   if (!aligned16(d_ckpt) || !aligned16(d_work))
     return fail(HS2_E_ARG, "hs2_grad_backward: d_ckpt and d_work must be 16-byte aligned");
-  const size_t need = (3 * (size_t)ckpt_every + 6) * (size_t)p->n;
+  const size_t need = hs2_grad_work_doubles(p, ckpt_every);
   if (work_doubles < need)
     return fail(HS2_E_ARG, "hs2_grad_backward: work buffer has %zu doubles, needs %zu",
                 work_doubles, need);

@@ -201,14 +201,17 @@ int hs2_run_timed(hs2_plan *plan, double *d_T, int nsteps, int method, double *k
  * ckpt_every steps.  Works in both coefficient modes; gradients with
  * respect to per-voxel parameters need hs2_plan_set_dense. */
 
-/* Doubles of device workspace for hs2_grad_backward: (3*ckpt_every+6)*n (each
- * segment's states T^n, T*, T** are recomputed once and kept) on class maps.
- * On per-voxel coefficients 7*n more, where sensitivities are added for four
- * steps at a time, and on small grids another (3*ckpt_every+1)*n, with which a
- * segment is recomputed on a second stream beside the adjoint steps of the one
- * after it.  hs2_grad_backward also takes the smaller ones and then does
- * without, with the same results. */
+/* Doubles of device workspace hs2_grad_backward needs: (3*ckpt_every+6)*n (each
+ * segment's states T^n, T*, T** are recomputed once and kept). */
 size_t hs2_grad_work_doubles(const hs2_plan *plan, int ckpt_every);
+
+/* Doubles of workspace with which a hs2_grad_backward of nsteps steps is
+ * fastest; the results have the same bits with any size from the least to this.
+ * On per-voxel coefficients 7*n more than the least, where sensitivities are
+ * added for four steps at a time, and on small grids with more than one segment
+ * another (3*ckpt_every+1)*n (up to 8 GiB), with which a segment is recomputed on
+ * a second stream beside the adjoint steps of the one after it. */
+size_t hs2_grad_work_best(const hs2_plan *plan, int nsteps, int ckpt_every);
 
 /* Forward pass: nsteps steps in place on d_T (T^0 in, T^nsteps out),
  * writing T^{k*ckpt_every} to d_ckpt + k*n (ceil(nsteps/ckpt_every) fields)
@@ -222,8 +225,8 @@ int hs2_grad_forward(hs2_plan *plan, double *d_T, int nsteps, int ckpt_every, do
  * plan coefficients, nsteps, ckpt_every and sources).  d_grad_hist: dJ/dhist
  * (nsteps x ny x nx).  Writes d_gM, d_gz, d_gy, d_gx (n each), d_gsrc
  * (nsrc x n; may be NULL when nsrc == 0) and, if not NULL, d_gT0 (n).
- * d_work: hs2_grad_work_doubles() doubles of scratch (or (3*ckpt_every+6)*n).
- * Needs nz >= 2 and every axis length <= 1024. */
+ * d_work: hs2_grad_work_doubles() doubles of scratch, or up to
+ * hs2_grad_work_best().  Needs nz >= 2 and every axis length <= 1024. */
 int hs2_grad_backward(hs2_plan *plan, int nsteps, int ckpt_every, const double *d_ckpt,
                       const double *d_src, const int32_t *h_src_step, int nsrc,
                       const double *d_grad_hist, double *d_gM, double *d_gz, double *d_gy,
