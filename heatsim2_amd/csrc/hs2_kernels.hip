@@ -1135,13 +1135,14 @@ static hipError_t launch_s_v(SConfig cfg, const Grid &g, const V &v, int axis, c
                              const double *Y, double *X, double *surf, double dz, bool ry,
                              hipStream_t s) {
   // per-voxel columns come here beyond 512 cells, where P x CW <= 512 with CW
-  // >= 8 leaves segments of 16 and more
+  // >= 8 leaves segments of 16 and more, and in fields of 4 GiB and more, whose
+  // axes are no shorter than 512: 8 cells x 8 lines serve those exactly
   if constexpr (std::is_same<V, ClassView>::value) {
     if (cfg.seg == 2) return launch_s_t<V, 2>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     if (cfg.seg == 4) return launch_s_t<V, 4>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
-    if (cfg.seg == 8) return launch_s_t<V, 8>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
   }
   switch (cfg.seg) {
+    case 8: return launch_s_t<V, 8>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     case 16: return launch_s_t<V, 16>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     case 32: return launch_s_t<V, 32>(g, v, axis, cfg.cw, Tn, Y, X, surf, dz, ry, s);
     default: return hipErrorInvalidValue;
