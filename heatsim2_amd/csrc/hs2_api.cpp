@@ -645,13 +645,24 @@ int without_lines(hs2_plan *p) {
   return p->mode == MODE_CLASS && !p->tried_comb ? build_combined(p) : HS2_OK;
 }
 
+// A device array of a function's own, freed however it is left.
+template <class T>
+struct DeviceArray {
+  T *p = nullptr;
+  DeviceArray() = default;
+  DeviceArray(const DeviceArray &) = delete;
+  DeviceArray &operator=(const DeviceArray &) = delete;
+  ~DeviceArray() { (void)hipFree(p); }
+  hipError_t alloc(size_t n) { return hipMalloc(&p, sizeof(T) * n); }
+};
+
 // Device copy of `v`, owned by the plan's line tables.
 template <class T>
 hipError_t keep_lines(hs2_plan *p, const std::vector<T> &v, const T **out) {
-  void *d = nullptr;
+  p->d_lines.push_back(nullptr);  // the slot first: it may throw
+  void *&d = p->d_lines.back();
   hipError_t e = hipMalloc(&d, sizeof(T) * std::max<size_t>(v.size(), 1));
   if (e != hipSuccess) return e;
-  p->d_lines.push_back(d);
   *out = static_cast<const T *>(d);
   return v.empty() ? hipSuccess
                    : hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
@@ -665,67 +676,60 @@ hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
                           std::vector<uint8_t> *bytes, int *count) {
   const hs2::Grid g = grid_of(p);
   const uint8_t *cz = p->cv.cls[0], *cy = p->cv.cls[1], *cx = p->cv.cls[2];
-  unsigned long long *d_hash = nullptr;
-  int *d_rep = nullptr;
-  uint8_t *d_bytes = nullptr;
+  DeviceArray<unsigned long long> d_hash;
+  DeviceArray<int> d_rep;
+  DeviceArray<uint8_t> d_bytes;
   *count = 0;
   std::vector<unsigned long long> h(2 * (size_t)lines);
-  auto run = [&]() -> hipError_t {
-    hipError_t e = hipMalloc(&d_hash, sizeof(h[0]) * h.size());
-    if (e == hipSuccess) e = hs2::launch_line_hash(g, cz, cy, cx, which, d_hash, 0);
-    if (e == hipSuccess)
-      e = hipMemcpy(h.data(), d_hash, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return e;
-    struct Key {
-      unsigned long long a, b;
-      bool operator==(const Key &o) const { return a == o.a && b == o.b; }
-    };
-    struct Hash {
-      size_t operator()(const Key &k) const { return (size_t)(k.a ^ (k.b >> 7)); }
-    };
-    std::unordered_map<Key, int, Hash> seen;
-    id->assign(lines, 0);
-    first->clear();
-    std::vector<int> rep(lines);
-    for (int ln = 0; ln < lines; ln++) {
-      const Key k{h[2 * (size_t)ln], h[2 * (size_t)ln + 1]};
-      int i;
-      if (ln > 0 && k == Key{h[2 * (size_t)ln - 2], h[2 * (size_t)ln - 1]}) {
-        i = (*id)[ln - 1];
-      } else {
-        auto it = seen.find(k);
-        if (it == seen.end()) {
-          if ((int)first->size() == most) return hipSuccess;
-          it = seen.emplace(k, (int)first->size()).first;
-          first->push_back(ln);
-        }
-        i = it->second;
-      }
-      (*id)[ln] = i;
-      rep[ln] = (*first)[i];
-    }
-    const int cnt = (int)first->size();
-    bytes->resize((size_t)cnt * len);
-    int flag = 0;
-    if ((e = hipMalloc(&d_rep, sizeof(int) * ((size_t)lines + cnt + 1))) != hipSuccess) return e;
-    int *d_first = d_rep + lines, *d_flag = d_first + cnt;
-    if ((e = hipMemcpy(d_rep, rep.data(), sizeof(int) * lines, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(d_first, first->data(), sizeof(int) * cnt, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(d_flag, &flag, sizeof flag, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMalloc(&d_bytes, bytes->size())) != hipSuccess ||
-        (e = hs2::launch_line_check(g, cz, cy, cx, which, d_rep, d_flag, 0)) != hipSuccess ||
-        (e = hs2::launch_line_gather(g, cz, cy, cx, which, d_first, cnt, d_bytes, 0)) != hipSuccess ||
-        (e = hipMemcpy(&flag, d_flag, sizeof flag, hipMemcpyDeviceToHost)) != hipSuccess ||
-        (e = hipMemcpy(bytes->data(), d_bytes, bytes->size(), hipMemcpyDeviceToHost)) != hipSuccess)
-      return e;
-    if (!flag) *count = cnt;
-    return hipSuccess;
+  hipError_t e = d_hash.alloc(h.size());
+  if (e == hipSuccess) e = hs2::launch_line_hash(g, cz, cy, cx, which, d_hash.p, 0);
+  if (e == hipSuccess)
+    e = hipMemcpy(h.data(), d_hash.p, sizeof(h[0]) * h.size(), hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  struct Key {
+    unsigned long long a, b;
+    bool operator==(const Key &o) const { return a == o.a && b == o.b; }
   };
-  const hipError_t e = run();
-  (void)hipFree(d_hash);
-  (void)hipFree(d_rep);
-  (void)hipFree(d_bytes);
-  return e;
+  struct Hash {
+    size_t operator()(const Key &k) const { return (size_t)(k.a ^ (k.b >> 7)); }
+  };
+  std::unordered_map<Key, int, Hash> seen;
+  id->assign(lines, 0);
+  first->clear();
+  std::vector<int> rep(lines);
+  for (int ln = 0; ln < lines; ln++) {
+    const Key k{h[2 * (size_t)ln], h[2 * (size_t)ln + 1]};
+    int i;
+    if (ln > 0 && k == Key{h[2 * (size_t)ln - 2], h[2 * (size_t)ln - 1]}) {
+      i = (*id)[ln - 1];
+    } else {
+      auto it = seen.find(k);
+      if (it == seen.end()) {
+        if ((int)first->size() == most) return hipSuccess;
+        it = seen.emplace(k, (int)first->size()).first;
+        first->push_back(ln);
+      }
+      i = it->second;
+    }
+    (*id)[ln] = i;
+    rep[ln] = (*first)[i];
+  }
+  const int cnt = (int)first->size();
+  bytes->resize((size_t)cnt * len);
+  int flag = 0;
+  if ((e = d_rep.alloc((size_t)lines + cnt + 1)) != hipSuccess) return e;
+  int *d_first = d_rep.p + lines, *d_flag = d_first + cnt;
+  if ((e = hipMemcpy(d_rep.p, rep.data(), sizeof(int) * lines, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = hipMemcpy(d_first, first->data(), sizeof(int) * cnt, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = hipMemcpy(d_flag, &flag, sizeof flag, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = d_bytes.alloc(bytes->size())) != hipSuccess ||
+      (e = hs2::launch_line_check(g, cz, cy, cx, which, d_rep.p, d_flag, 0)) != hipSuccess ||
+      (e = hs2::launch_line_gather(g, cz, cy, cx, which, d_first, cnt, d_bytes.p, 0)) != hipSuccess ||
+      (e = hipMemcpy(&flag, d_flag, sizeof flag, hipMemcpyDeviceToHost)) != hipSuccess ||
+      (e = hipMemcpy(bytes->data(), d_bytes.p, bytes->size(), hipMemcpyDeviceToHost)) != hipSuccess)
+    return e;
+  if (!flag) *count = cnt;
+  return hipSuccess;
 }
 
 // Line tables of the plan's axes (hs2_lines.h), where they pay:
@@ -1005,10 +1009,10 @@ int hs2_plan_set_compact(hs2_plan *p, const uint8_t *d_mat, const uint8_t *d_bz,
     p->cv.tab = p->d_tab;
     for (int t = 0; t < 4; t++) p->cv.off[t] = off[t];
     p->mode = MODE_CLASS;
-    p->tabs = tabs;
+    p->tabs.swap(tabs);
     hipError_t e = hipSuccess;
     try {
-      e = build_lines(p, tabs, off);
+      e = build_lines(p, p->tabs, off);
     } catch (const std::bad_alloc &) {
       e = hipErrorOutOfMemory;
     }
