@@ -575,76 +575,6 @@ int batch_lanes(hs2_batch *b, int reset, Turns turns, Turn turn) {
   return HS2_OK;
 }
 
-// The x sweep's combined class plane: one id per cell for its (z, y, x)
-// class triple, when the triples number 256 or fewer (else the x sweep
-// reads the three class planes).
-int build_combined(hs2_plan *p) {
-  const std::vector<double> &tabs = p->tabs;
-  const int *off = p->cv.off;
-  p->tried_comb = true;
-  constexpr size_t kWords = (size_t(1) << 24) / 32;
-  const int n = p->n;
-  const uint8_t *cz = p->cv.cls[0], *cy = p->cv.cls[1], *cx = p->cv.cls[2];
-  uint32_t *d_bits = nullptr;
-  int *d_rank = nullptr;
-  std::vector<uint32_t> bits(kWords);
-  std::vector<int> rank0(kWords);
-  std::vector<uint32_t> keys;
-  auto done = [&](int rc) {
-    (void)hipFree(d_bits);
-    (void)hipFree(d_rank);
-    return rc;
-  };
-  hipError_t e = hipMalloc(&d_bits, kWords * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemset(d_bits, 0, kWords * sizeof(uint32_t));
-  if (e == hipSuccess) e = hs2::launch_comb_mark(n, cz, cy, cx, d_bits, 0);
-  if (e == hipSuccess)
-    e = hipMemcpy(bits.data(), d_bits, kWords * sizeof(uint32_t), hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return done(fail(HS2_E_HIP, "combined class plane: %s", hipGetErrorString(e)));
-  int cnt = 0;
-  for (size_t w = 0; w < kWords; w++) {
-    rank0[w] = cnt;
-    for (uint32_t b = bits[w]; b; b &= b - 1, cnt++)
-      keys.push_back((uint32_t)(w * 32 + __builtin_ctz(b)));
-  }
-  if (cnt > hs2::kMaxClass) return done(HS2_OK);  // the three planes serve
-  std::vector<double> ctab((size_t)hs2::CombView::kStride * cnt, 0.0);
-  for (int i = 0; i < cnt; i++) {
-    const uint32_t id[3] = {keys[i] & 0xffu, (keys[i] >> 8) & 0xffu, keys[i] >> 16};  // z, y, x
-    for (int a = 0; a < 3; a++) {
-      const double *src = &tabs[off[a] + (size_t)id[a] * hs2::kTabStride];
-      double *dst = &ctab[(size_t)i * hs2::CombView::kStride + 4 * (2 - a)];
-      for (int k = 0; k < 3; k++) dst[k] = src[k];
-    }
-  }
-  e = hipMalloc(&d_rank, kWords * sizeof(int));
-  if (e == hipSuccess) e = hipMemcpy(d_rank, rank0.data(), kWords * sizeof(int), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&p->d_comb, (size_t)n);
-  if (e == hipSuccess) e = hipMalloc(&p->d_ctab, sizeof(double) * ctab.size());
-  if (e == hipSuccess)
-    e = hipMemcpy(p->d_ctab, ctab.data(), sizeof(double) * ctab.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hs2::launch_comb_assign(n, cz, cy, cx, d_bits, d_rank, p->d_comb, 0);
-  if (e == hipSuccess) e = hipDeviceSynchronize();
-  if (e != hipSuccess) {
-    (void)hipFree(p->d_comb);
-    (void)hipFree(p->d_ctab);
-    p->d_comb = nullptr;
-    p->d_ctab = nullptr;
-    return done(fail(HS2_E_HIP, "combined class plane: %s", hipGetErrorString(e)));
-  }
-  p->comb.comb = p->d_comb;
-  p->comb.tab = p->d_ctab;
-  p->comb.n = cnt;
-  p->have_comb = true;
-  return done(HS2_OK);
-}
-
-// The combined plane, which only an x sweep without line tables reads: built
-// when a plan is left without them (1.3 ms at 40^3, of 3.0 for the whole set-up).
-int without_lines(hs2_plan *p) {
-  return p->mode == MODE_CLASS && !p->tried_comb ? build_combined(p) : HS2_OK;
-}
-
 // A device array of a function's own, freed however it is left.
 template <class T>
 struct DeviceArray {
@@ -655,6 +585,83 @@ struct DeviceArray {
   ~DeviceArray() { (void)hipFree(p); }
   hipError_t alloc(size_t n) { return hipMalloc(&p, sizeof(T) * n); }
 };
+
+// The x sweep's combined class plane: one id per cell for its (z, y, x)
+// class triple, when the triples number 256 or fewer (else the x sweep
+// reads the three class planes).
+hipError_t build_combined(hs2_plan *p) {
+  const std::vector<double> &tabs = p->tabs;
+  const int *off = p->cv.off;
+  constexpr size_t kWords = (size_t(1) << 24) / 32;
+  const int n = p->n;
+  const uint8_t *cz = p->cv.cls[0], *cy = p->cv.cls[1], *cx = p->cv.cls[2];
+  DeviceArray<uint32_t> d_bits;
+  DeviceArray<int> d_rank;
+  DeviceArray<uint8_t> d_comb;
+  DeviceArray<double> d_ctab;
+  std::vector<uint32_t> bits(kWords);
+  std::vector<int> rank0(kWords);
+  std::vector<uint32_t> keys;
+  hipError_t e = d_bits.alloc(kWords);
+  if (e == hipSuccess) e = hipMemset(d_bits.p, 0, kWords * sizeof(uint32_t));
+  if (e == hipSuccess) e = hs2::launch_comb_mark(n, cz, cy, cx, d_bits.p, 0);
+  if (e == hipSuccess)
+    e = hipMemcpy(bits.data(), d_bits.p, kWords * sizeof(uint32_t), hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  int cnt = 0;
+  for (size_t w = 0; w < kWords; w++) {
+    rank0[w] = cnt;
+    for (uint32_t b = bits[w]; b; b &= b - 1, cnt++)
+      keys.push_back((uint32_t)(w * 32 + __builtin_ctz(b)));
+  }
+  if (cnt > hs2::kMaxClass) {  // the three planes serve
+    p->tried_comb = true;
+    return hipSuccess;
+  }
+  std::vector<double> ctab((size_t)hs2::CombView::kStride * cnt, 0.0);
+  for (int i = 0; i < cnt; i++) {
+    const uint32_t id[3] = {keys[i] & 0xffu, (keys[i] >> 8) & 0xffu, keys[i] >> 16};  // z, y, x
+    for (int a = 0; a < 3; a++) {
+      const double *src = &tabs[off[a] + (size_t)id[a] * hs2::kTabStride];
+      double *dst = &ctab[(size_t)i * hs2::CombView::kStride + 4 * (2 - a)];
+      for (int k = 0; k < 3; k++) dst[k] = src[k];
+    }
+  }
+  e = d_rank.alloc(kWords);
+  if (e == hipSuccess) e = hipMemcpy(d_rank.p, rank0.data(), kWords * sizeof(int), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = d_comb.alloc((size_t)n);
+  if (e == hipSuccess) e = d_ctab.alloc(ctab.size());
+  if (e == hipSuccess)
+    e = hipMemcpy(d_ctab.p, ctab.data(), sizeof(double) * ctab.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hs2::launch_comb_assign(n, cz, cy, cx, d_bits.p, d_rank.p, d_comb.p, 0);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e != hipSuccess) return e;
+  std::swap(p->d_comb, d_comb.p);
+  std::swap(p->d_ctab, d_ctab.p);
+  p->comb.comb = p->d_comb;
+  p->comb.tab = p->d_ctab;
+  p->comb.n = cnt;
+  p->have_comb = p->tried_comb = true;
+  return hipSuccess;
+}
+
+// The combined plane, which only an x sweep without line tables reads: built
+// when a plan is left without them (1.3 ms at 40^3, of 3.0 for the whole set-up).
+// Without the memory for it the three planes serve.
+int without_lines(hs2_plan *p) {
+  if (p->mode != MODE_CLASS || p->tried_comb) return HS2_OK;
+  hipError_t e;
+  try {
+    e = build_combined(p);
+  } catch (const std::bad_alloc &) {
+    e = hipErrorOutOfMemory;
+  }
+  if (e == hipSuccess) return HS2_OK;
+  (void)hipGetLastError();
+  return e == hipErrorOutOfMemory
+             ? HS2_OK
+             : fail(HS2_E_HIP, "combined class plane: %s", hipGetErrorString(e));
+}
 
 // Device copy of `v`, owned by the plan's line tables.
 template <class T>

@@ -130,7 +130,10 @@ int hs2_plan_set_config(hs2_plan *plan, int x_cpl, int x_lanes, int x_lines, int
  *     its shapes are the other kernels'): with class maps, sweep the axes
  *     whose lines fall into few distinct ones with those lines' factors,
  *     computed once by hs2_plan_set_compact; 0 eliminates every line from
- *     its class bytes on every step.  Same steps to round-off. */
+ *     its class bytes on every step.  Same steps to round-off.
+ * Switching line tables off (0, or hs2_plan_set_config) builds the combined
+ * plane the first time, where there is memory for it: it allocates and
+ * synchronises then. */
 enum { HS2_OPT_COMBINED_X = 1, HS2_OPT_LINE_TABLES = 2 };
 int hs2_plan_set_option(hs2_plan *plan, int option, int value);
 

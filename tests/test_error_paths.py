@@ -32,7 +32,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["set_compact_host_memory", "set_compact_device_memory"])
+@pytest.mark.parametrize("what", ["set_compact_host_memory", "set_compact_device_memory",
+                                  "set_config_host_memory", "set_config_device_memory"])
 def test_error_path(program, what):
     run = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout[-2000:] + run.stderr[-2000:]
