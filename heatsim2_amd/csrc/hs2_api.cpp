@@ -539,15 +539,53 @@ int batch_replay(hs2_batch *b, hipStream_t s, hipGraphExec_t *exec, std::vector<
   return HS2_OK;
 }
 
+// The batch's own streams between a call's first work on them and its return:
+// they begin after the caller's stream, and however the call ends, the caller's
+// stream comes after them.
+struct BatchStreams {
+  hs2_batch *b;
+  hipStream_t stream;
+  bool open = false;
+  BatchStreams(hs2_batch *batch, hipStream_t s) : b(batch), stream(s) {}
+  ~BatchStreams() {
+    if (open) (void)join();
+  }
+  hipError_t begin() {
+    hipError_t e = hipEventRecord(b->ev_in, stream);
+    open = e == hipSuccess;
+    return open ? hipStreamWaitEvent(b->stream[0], b->ev_in, 0) : e;
+  }
+  // the other lanes start after what the first has so far
+  hipError_t fork() {
+    hipError_t e = hipEventRecord(b->ev_lane, b->stream[0]);
+    for (int lane = 1; lane < kBatchLanes && e == hipSuccess; lane++)
+      if (b->stream[lane]) e = hipStreamWaitEvent(b->stream[lane], b->ev_lane, 0);
+    return e;
+  }
+  hipError_t join() {
+    open = false;
+    hipError_t first = hipSuccess;
+    for (int lane = kBatchLanes - 1; lane >= 0; lane--) {
+      if (!b->stream[lane]) continue;
+      const hipEvent_t ev = lane ? b->ev_lane : b->ev_out;
+      hipError_t e = hipEventRecord(ev, b->stream[lane]);
+      if (e == hipSuccess) e = hipStreamWaitEvent(lane ? b->stream[0] : stream, ev, 0);
+      if (e != hipSuccess) {
+        (void)hipStreamSynchronize(b->stream[lane]);
+        if (first == hipSuccess) first = e;
+      }
+    }
+    return first;
+  }
+};
+
 // Every group's turns on its lane's stream, the lanes in turn so that all of
-// them have work at once; then the first lane waits for the others.  reset:
-// the counter that a group starts from 0; turns(g), turn(g).
+// them have work at once.  reset: the counter that a group starts from 0;
+// turns(g), turn(g).
 template <class Turns, class Turn>
 int batch_lanes(hs2_batch *b, int reset, Turns turns, Turn turn) {
   size_t at[kBatchLanes] = {};
   int done[kBatchLanes] = {};
-  for (int lane = 1; lane < kBatchLanes; lane++)
-    if (b->stream[lane]) HIP_TRY(hipStreamWaitEvent(b->stream[lane], b->ev_lane, 0));
   for (bool any = true; any;) {
     any = false;
     for (int lane = 0; lane < kBatchLanes; lane++) {
@@ -567,11 +605,6 @@ int batch_lanes(hs2_batch *b, int reset, Turns turns, Turn turn) {
       }
     }
   }
-  for (int lane = 1; lane < kBatchLanes; lane++)
-    if (b->stream[lane]) {
-      HIP_TRY(hipEventRecord(b->ev_lane, b->stream[lane]));
-      HIP_TRY(hipStreamWaitEvent(b->stream[0], b->ev_lane, 0));
-    }
   return HS2_OK;
 }
 
@@ -1703,9 +1736,9 @@ int hs2_batch_forward(hs2_batch *b, double *d_T, const double *d_src, double *d_
   if (work_doubles < (size_t)batch_work_doubles(b))
     return fail(HS2_E_ARG, "hs2_batch_forward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
-  HIP_TRY(hipEventRecord(b->ev_in, (hipStream_t)stream));
-  HIP_TRY(hipStreamWaitEvent(b->stream[0], b->ev_in, 0));
-  HIP_TRY(hipEventRecord(b->ev_lane, b->stream[0]));
+  BatchStreams streams(b, (hipStream_t)stream);
+  HIP_TRY(streams.begin());
+  HIP_TRY(streams.fork());
   auto chunk = [&](const batch_group &g) { return std::min(b->chunk, g.maxsteps); };
   const int rc = batch_lanes(
       b, 0, [&](const batch_group &g) { return (g.maxsteps + chunk(g) - 1) / chunk(g); },
@@ -1720,8 +1753,7 @@ int hs2_batch_forward(hs2_batch *b, double *d_T, const double *d_src, double *d_
             "hs2_batch_forward");
       });
   if (rc != HS2_OK) return rc;
-  HIP_TRY(hipEventRecord(b->ev_out, b->stream[0]));
-  HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
+  HIP_TRY(streams.join());
   return HS2_OK;
 }
 
@@ -1735,8 +1767,8 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
     return fail(HS2_E_ARG, "hs2_batch_backward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
   hipStream_t s = b->stream[0];
-  HIP_TRY(hipEventRecord(b->ev_in, (hipStream_t)stream));
-  HIP_TRY(hipStreamWaitEvent(s, b->ev_in, 0));
+  BatchStreams streams(b, (hipStream_t)stream);
+  HIP_TRY(streams.begin());
   HIP_TRY(hs2::launch_fill(d_gM, b->N, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gz, b->N, 0.0, s));
   HIP_TRY(hs2::launch_fill(d_gy, b->N, 0.0, s));
@@ -1745,7 +1777,7 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   const std::vector<const void *> key = {d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc,
                                          d_work, b->dv.M, b->dv.w, b->dv.g[0], b->dv.g[1],
                                          b->dv.g[2]};
-  HIP_TRY(hipEventRecord(b->ev_lane, s));
+  HIP_TRY(streams.fork());
   const int rc = batch_lanes(
       b, 1, [&](const batch_group &g) { return (g.maxsteps + b->K - 1) / b->K; },
       [&](batch_group &g, hipStream_t st) {
@@ -1758,8 +1790,7 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
             "hs2_batch_backward");
       });
   if (rc != HS2_OK) return rc;
-  HIP_TRY(hipEventRecord(b->ev_out, s));
-  HIP_TRY(hipStreamWaitEvent((hipStream_t)stream, b->ev_out, 0));
+  HIP_TRY(streams.join());
   return HS2_OK;
 }
 

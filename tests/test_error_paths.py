@@ -33,7 +33,8 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("what", ["set_compact_host_memory", "set_compact_device_memory",
-                                  "set_config_host_memory", "set_config_device_memory"])
+                                  "set_config_host_memory", "set_config_device_memory",
+                                  "batch_lanes", "batch_lanes_graphs", "backward_lanes"])
 def test_error_path(program, what):
     run = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout[-2000:] + run.stderr[-2000:]
