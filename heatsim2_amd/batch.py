@@ -86,8 +86,13 @@ class GradBatch(object):
 
     def work(self):
         if self._work is None:
-            self._work = torch.empty(self.work_doubles, dtype=torch.float64,
-                                     device=_lib.device())
+            try:
+                self._work = torch.empty(self.work_doubles, dtype=torch.float64,
+                                         device=_lib.device())
+            except torch.cuda.OutOfMemoryError:  # the least that the calls take
+                self.work_doubles -= 8 * self.N
+                self._work = torch.empty(self.work_doubles, dtype=torch.float64,
+                                         device=_lib.device())
         return self._work
 
     def run(self, coefs, T0s, srcs=None):

@@ -414,12 +414,18 @@ void batch_free(hs2_batch *b) {
 }
 
 // work layout: ws (N) | checkpoints (CK) | segment T^t (K+1 N) | T* (K N) | T** (K N) |
-// u_z u_y u_x of each step of a group (3 N each)
+// u_z u_y u_x of each step of a group (3 N each; a group has as many steps, up to
+// kAdjGroup, as the buffer has room for, and at least one)
 struct BatchWork {
   double *ws, *ck, *seg, *segx, *segy, *u;
 };
 long long batch_work_doubles(const hs2_batch *b) {
   return b->N * (3LL * b->K + 2 + 3 * hs2::kAdjGroup) + b->CK;
+}
+long long batch_work_least(const hs2_batch *b) { return b->N * (3LL * b->K + 6) + b->CK; }
+int batch_adj_group(const hs2_batch *b, size_t work_doubles) {
+  const long long left = (long long)work_doubles - b->CK - b->N * (3LL * b->K + 2);
+  return (int)std::min<long long>(hs2::kAdjGroup, left / (3 * b->N));
 }
 BatchWork batch_work(const hs2_batch *b, double *w) {
   BatchWork r;
@@ -455,7 +461,7 @@ hipError_t emit_forward(hs2_batch *b, const batch_group &g, double *T, const dou
 hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const double *src,
                                  const double *ghist,
                                  double *gM, double *gz, double *gy, double *gx, double *gsrc,
-                                 const BatchWork &w, hipStream_t s) {
+                                 const BatchWork &w, int S, hipStream_t s) {
   const int K = b->K;
   const size_t N = (size_t)b->N;
   hipError_t e = hs2::launch_batch_ckpt_load(batch_map(b, g, KIND_CELL, hs2::RULE_SEG, 0),
@@ -475,7 +481,6 @@ hipError_t emit_backward_segment(hs2_batch *b, const batch_group &g, const doubl
   // adjoint steps, latest first: lambda from the solves of the step after (the
   // last one of the segment before has slot (K - 1) % S) and the z, y, x
   // transposed solves; the sensitivities group by group
-  constexpr int S = hs2::kAdjGroup;
   for (int j = 0; j < K && e == hipSuccess; j++) {
     double *uz = w.u + (size_t)(j % S) * 3 * N, *uy = uz + N, *ux = uy + N;
     const double *after = w.u + (size_t)((j > 0 ? j - 1 : K - 1) % S) * 3 * N;
@@ -1733,7 +1738,7 @@ int hs2_batch_forward(hs2_batch *b, double *d_T, const double *d_src, double *d_
   if (!b->have_coef) return fail(HS2_E_STATE, "hs2_batch_forward: coefficients not set");
   if (!aligned16(d_T) || !aligned16(d_work) || (d_src && !aligned16(d_src)))
     return fail(HS2_E_ARG, "hs2_batch_forward: fields must be 16-byte aligned");
-  if (work_doubles < (size_t)batch_work_doubles(b))
+  if (work_doubles < (size_t)batch_work_least(b))
     return fail(HS2_E_ARG, "hs2_batch_forward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
   BatchStreams streams(b, (hipStream_t)stream);
@@ -1763,9 +1768,10 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   if (!b || !d_grad_hist || !d_gM || !d_gz || !d_gy || !d_gx || !d_work)
     return fail(HS2_E_ARG, "hs2_batch_backward: null argument");
   if (!b->have_coef) return fail(HS2_E_STATE, "hs2_batch_backward: coefficients not set");
-  if (work_doubles < (size_t)batch_work_doubles(b))
+  if (work_doubles < (size_t)batch_work_least(b))
     return fail(HS2_E_ARG, "hs2_batch_backward: work buffer too small");
   const BatchWork w = batch_work(b, d_work);
+  const int S = batch_adj_group(b, work_doubles);
   hipStream_t s = b->stream[0];
   BatchStreams streams(b, (hipStream_t)stream);
   HIP_TRY(streams.begin());
@@ -1776,7 +1782,7 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
   if (d_gsrc) HIP_TRY(hs2::launch_fill(d_gsrc, b->N, 0.0, s));
   const std::vector<const void *> key = {d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx, d_gsrc,
                                          d_work, b->dv.M, b->dv.w, b->dv.g[0], b->dv.g[1],
-                                         b->dv.g[2]};
+                                         b->dv.g[2], (const void *)(intptr_t)S};
   HIP_TRY(streams.fork());
   const int rc = batch_lanes(
       b, 1, [&](const batch_group &g) { return (g.maxsteps + b->K - 1) / b->K; },
@@ -1785,7 +1791,7 @@ int hs2_batch_backward(hs2_batch *b, const double *d_src, const double *d_grad_h
             b, st, &g.bwd_exec, &g.bwd_key, key,
             [&](hipStream_t s) {
               return emit_backward_segment(b, g, d_src, d_grad_hist, d_gM, d_gz, d_gy, d_gx,
-                                           d_gsrc, w, s);
+                                           d_gsrc, w, S, s);
             },
             "hs2_batch_backward");
       });

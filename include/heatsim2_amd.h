@@ -262,7 +262,9 @@ void hs2_batch_destroy(hs2_batch *batch);
  * instance in the concatenated fields and first value of its surface
  * history (nsteps x ny x nx); the last entries are the totals.  sizes[5]
  * (may be NULL): total cells, total history values, work doubles,
- * checkpoint interval, largest step count. */
+ * checkpoint interval, largest step count.  8 doubles of work less per cell do
+ * as well: sensitivities are then added step by step, not four at a time, to the
+ * same bits. */
 int hs2_batch_layout(const hs2_batch *batch, int64_t *cell_off, int64_t *hist_off,
                      int64_t *sizes);
 

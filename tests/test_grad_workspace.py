@@ -1,10 +1,10 @@
-"""The scratch of hs2_grad_backward: what the library asks for, what
-surface_history takes, and what it falls back to when memory is short."""
+"""The scratch of the gradients, of one plan and of a batch: what the library
+asks for, what the package takes, and what it falls back to when memory is short."""
 import numpy as np
 import pytest
 import torch
 
-from heatsim2_amd import _lib, adjoint
+from heatsim2_amd import _lib, adjoint, batch
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +94,49 @@ def test_short_memory(room):
         torch.cuda.set_per_process_memory_fraction(1.0)
     got = [coef[name].grad.cpu() for name in ("M", "gz", "gy", "gx")]
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("every", [2, 6])
+def test_batches_in_short_memory(every):
+    """A batch whose scratch lacks the 8 fields that sensitivities four steps at a
+    time take: the same bits; and one field less is refused."""
+    torch.cuda.empty_cache()
+    shapes, steps = [(40, 64, 64), (64, 50, 70), (33, 65, 90)], [5, 9, 14]
+    rng = np.random.default_rng(every)
+    up = lambda a: torch.from_numpy(a).cuda()
+    coefs, T0s, Gs = [], [], []
+    for shape, n in zip(shapes, steps):
+        c = dict(M=up(1.0 + rng.random(shape)), w=torch.ones(shape, dtype=torch.uint8, device="cuda"))
+        for a, name in enumerate(("gz", "gy", "gx")):
+            c[name] = up(0.5 * rng.random(shape))
+            c[name].select(a, 0).zero_()
+        coefs.append(c)
+        T0s.append(up(rng.random(shape)))
+        Gs.append(up(rng.random((n,) + shape[1:])))
+
+    def gradients(gb):
+        leaves = [{k: v.clone().requires_grad_() if k != "w" else v for k, v in c.items()}
+                  for c in coefs]
+        h = gb.surface_history(leaves, T0s)
+        sum((a * G).sum() for a, G in zip(h, Gs)).backward()
+        torch.cuda.synchronize()
+        return [c[k].grad.cpu() for c in leaves for k in ("M", "gz", "gy", "gx")]
+
+    want = gradients(batch.GradBatch(shapes, [1e-3] * 3, steps, [-1] * 3, ckpt_every=every))
+    gb = batch.GradBatch(shapes, [1e-3] * 3, steps, [-1] * 3, ckpt_every=every)
+    full = gb.work_doubles
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction(
+            (torch.cuda.memory_reserved() + (full - 4 * gb.N) * 8) / total)
+        gb.work()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert gb.work_doubles == full - 8 * gb.N == gb._work.numel()
+    got = gradients(gb)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    gb.work_doubles -= gb.N
+    with pytest.raises(_lib.HS2Error):
+        gradients(gb)
