@@ -66,6 +66,7 @@ struct hs2_plan {
   // line tables (class mode): the axes whose distinct lines are factored
   bool use_lines = true;        // hs2_plan_set_option(HS2_OPT_LINE_TABLES)
   hs2::RowTab rows{};           // x; g = 0: none
+  bool rows_plain = false;      // in steps without sources too
   hs2::ColTab cols[2] = {};     // [0] z, [1] y; P = 0: none
   std::vector<void *> d_lines;  // their device arrays
   hs2::DenseView dv{};
@@ -217,10 +218,15 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 hs2::Grid grid_of(const hs2_plan *p) { return hs2::Grid{p->grid.nz, p->grid.ny, p->grid.nx}; }
 
+// whether the x sweep of a step (src: with sources) runs on line tables
+bool row_tables(const hs2_plan *p, bool src) {
+  return p->use_lines && p->rows.g && (src || p->rows_plain);
+}
+
 hipError_t sweep_x(const hs2_plan *p, const double *Tn, double *Ts, const uint8_t *vmap,
                    const double *vtab, const double *sfield, hipStream_t s, bool ry = false) {
   const hs2::Grid g = grid_of(p);
-  if (p->use_lines && p->rows.g)
+  if (row_tables(p, vmap || sfield))
     return hs2::launch_rows(g, p->rows, Tn, Ts, vmap, vtab, sfield, ry, s);
   if (p->mode == MODE_CLASS && p->have_comb && p->use_comb && !vmap && !sfield &&
       hs2::x_ry_ok(p->xcfg, g))
@@ -250,7 +256,7 @@ hipError_t sweep_s(const hs2_plan *p, int axis, const double *Tn, const double *
 // read less) where the plan and the step allow it (on line tables always, on
 // per-voxel coefficients by the grid)
 bool use_ry(const hs2_plan *p, bool src) {
-  if (p->use_lines && p->rows.g) return true;
+  if (row_tables(p, src)) return true;
   if (p->mode == MODE_DENSE || p->mode == MODE_ASYM) return hs2::dense_ry(grid_of(p));
   return p->mode == MODE_CLASS && !src && hs2::x_ry_ok(p->xcfg, grid_of(p));
 }
@@ -347,6 +353,7 @@ void free_lines(hs2_plan *p) {
   for (void *d : p->d_lines) (void)hipFree(d);
   p->d_lines.clear();
   p->rows = hs2::RowTab{};
+  p->rows_plain = false;
   p->cols[0] = p->cols[1] = hs2::ColTab{};
 }
 
@@ -786,12 +793,36 @@ hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
 //                kernel);
 //   kMostVarying the share of rows whose explicit numbers vary along them,
 //                kMostCells the bytes of those numbers (61 x 149 x 203: x
-//                12.6 us without such rows, 17.8 with them all around, 21.6
-//                with them in two planes of three, against 25.8).
+//                15.3 us without such rows, 17.7 with half of them alike, 24.4
+//                with 32 MB of them, against 26.3 for the class kernel).  In
+//                rows of more than 512 cells a third is too much already
+//                (100 x 500 x 600: x 284 us at a fifth, 304 at 0.3, 325 at 0.4
+//                against 250; y, which has tables only with x's, gains 50).
+// Where the class kernel hands y its right-hand side too (x_ry_ok: whole lines of
+// 16-cell lanes), its source-free x sweep is half as fast again as where it
+// does not, and steps without sources use the tables only (rows_plain) with
+//   - kPlainCells bytes of such numbers at most, what an XCD's L2 holds (64 x
+//     128 x 256: x 12.3 us without, 14.7 with 5 MB, 16.4 with 10 and 19.6 with 30
+//     against 14.3; 48 x 200 x 512: 29.9, and 43.6 with 12, against 35.8),
+//   - a third of the rows varying at most (128 x 256 x 256: 36.5 at 0.3, 39.2 at
+//     0.4 against 37.4),
+//   - beyond 512 cells, where a line's factors (40 KB) come from L2 for every row,
+//     kPlainRows rows at most (1024 cells: a step 175 us at 16000 rows against 206
+//     with the class kernel's x, 269 at 20000 against 283, 455 at 31200 against
+//     435), and where any vary kPlainVarying (x 8.6 at 384 against 9.2, 11.2 at
+//     528 against 10.8, 51 at 7808 against 39; 81 at 16000 against 97, which is
+//     the exception).
+// Their source steps, for which that kernel has no such form, are faster on the
+// tables in all of these (by 1.0 to 1.5).
 hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int off[4]) {
   constexpr size_t kMostBytes = size_t(1) << 20, kMostCells = size_t(32) << 20;
   constexpr double kMostGroups = 1.35, kMostVarying = 0.5;
-  constexpr size_t kRowLds = 32768;  // of the rows' factors in LDS: four blocks per CU
+  constexpr size_t kPlainCells = size_t(4) << 20;
+  constexpr int kPlainRows = 20480, kPlainVarying = 448;
+  // of the rows' factors in LDS: four blocks per CU.  One line's at 385 to 512
+  // cells (the others' come from L2: two materials of 512 cells, 64 x 244 rows, x
+  // 35.3 us against 29.3 with one and 53 for the class kernel), none beyond.
+  constexpr size_t kRowLds = 32768;
   const hs2::Grid g = grid_of(p);
   if ((size_t)p->n * sizeof(double) >= (size_t(1) << 32)) return hipSuccess;
   std::vector<int> id, first, idx;
@@ -892,7 +923,7 @@ hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int o
     rid[r] |= eid[id[r]] << 16;
     varying += (eid[id[r]] & hs2::kRowVaries) != 0;
   }
-  if (varying > nrow * kMostVarying) return hipSuccess;
+  if (varying > nrow * (g.nx > 512 ? 0.3 : kMostVarying)) return hipSuccess;
   if ((e = keep_lines(p, lane, &t.lane)) != hipSuccess ||
       (e = keep_lines(p, row, &t.row)) != hipSuccess ||
       (e = keep_lines(p, cell, &t.cell)) != hipSuccess ||
@@ -902,6 +933,9 @@ hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int o
   t.nlds = (int)std::min<size_t>(lane.size() / ((size_t)rg * nc),
                                  kRowLds / (sizeof(double) * rg * nc));
   p->rows = t;
+  p->rows_plain = !hs2::x_ry_ok(p->xcfg, g) ||
+                  (sizeof(double) * cell.size() <= kPlainCells && 3 * varying <= nrow &&
+                   (g.nx <= 512 || nrow <= (varying ? kPlainVarying : kPlainRows)));
   return hipSuccess;
 }
 
@@ -1068,7 +1102,7 @@ int hs2_plan_set_compact(hs2_plan *p, const uint8_t *d_mat, const uint8_t *d_bz,
         return fail(HS2_E_HIP, "hs2_plan_set_compact: line tables: %s", hipGetErrorString(e));
       (void)hipGetLastError();
     }
-    return p->use_lines && p->rows.g ? HS2_OK : without_lines(p);
+    return row_tables(p, false) ? HS2_OK : without_lines(p);
   }
   // more than 256 classes on an axis: per-cell float64 coefficients
   double *d_gtab = nullptr, *d_mtab = nullptr;
@@ -1159,7 +1193,7 @@ int hs2_plan_info(const hs2_plan *p, int *info) {
   info[9] = p->scfg[0].cw;
   info[11] = p->xcfg.ty;
   info[12] = use_ry(p, false) ? 1 : 0;
-  info[13] = p->mode == MODE_CLASS && p->have_comb && p->use_comb &&
+  info[13] = p->mode == MODE_CLASS && !row_tables(p, false) && p->have_comb && p->use_comb &&
              hs2::x_ry_ok(p->xcfg, grid_of(p)) ? p->comb.n : 0;
   return HS2_OK;
 }

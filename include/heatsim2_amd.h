@@ -138,7 +138,8 @@ enum { HS2_OPT_COMBINED_X = 1, HS2_OPT_LINE_TABLES = 2 };
 int hs2_plan_set_option(hs2_plan *plan, int option, int value);
 
 /* An option's value; for HS2_OPT_LINE_TABLES the axes that are swept so
- * (1 x, 2 y, 4 z, added up; 0 when off). */
+ * (1 x, 2 y, 4 z, added up; 0 when off; x perhaps in steps with sources only,
+ * where the other kernel is the faster one without: info[13] is not 0 then). */
 int hs2_plan_get_option(const hs2_plan *plan, int option, int *value);
 
 /* info[0..13] = mode (0 none, 1 class maps, 2 dense, 3 dense per side),
