@@ -8,9 +8,10 @@ reduction across lanes / threads.  Candidates are timed on
 the device with HIP events (hs2_run_timed) on a scratch copy of the field;
 the fastest of each sweep is set on the plan.  These shapes are the class-map
 and per-cell kernels'; a plan with line tables (HS2_OPT_LINE_TABLES) is timed
-with them as well and keeps whichever is faster.  Results are cached per
+with them as well and keeps whichever is faster.  The shapes are cached per
 (device name, grid shape, coefficient mode) in memory and, if writable, in
-$HS2_TUNE_CACHE (default ~/.cache/heatsim2_amd/tune.json).
+$HS2_TUNE_CACHE (default ~/.cache/heatsim2_amd/tune.json); whether the tables are
+faster depends on the plan's maps and is timed for every plan.
 
 There is no upstream counterpart: the upstream solves every line with one
 serial Thomas pass (tridiag.pyx:46-69).
@@ -113,15 +114,16 @@ def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
     key = "%s|%s|%dx%dx%d|mode%d|lines%d" % (L.hs2_version().decode(),
                                              torch.cuda.get_device_name(), nz, ny, nx,
                                              info["mode"], lines)
+
+    def own_field():
+        return torch.full(ADI_params.shape, 293.0, dtype=torch.float64, device=_lib.device())
+
     if use_cache:
         cfg = _memo.get(key) or _load_cache().get(key)
         if cfg and _apply(L, plan, cfg, strict=False):
             _memo[key] = cfg
-            return cfg
-    dev = _lib.device()
-    if T is None:
-        T = torch.full(ADI_params.shape, 293.0, dtype=torch.float64, device=dev)
-    scratch = T.detach().clone()
+            return _with_lines(L, plan, cfg, own_field(), steps, verbose) if lines else dict(cfg)
+    scratch = own_field() if T is None else T.detach().clone()
     cur = {"x": (info["x_cpl"], info["x_lanes"], info["x_lines"], info["x_lines_y"]),
            "y": (info["y_seg"], info["y_lines"]),
            "z": (info["z_seg"], info["z_lines"])}
@@ -154,25 +156,28 @@ def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
         best_ms[idx] = _time(L, plan, scratch, steps)[idx] if results else None
     cfg = {"x": list(cur["x"]), "y": list(cur["y"]), "z": list(cur["z"]), "ms": best_ms,
            "lines": False}
-    if lines:
-        # each side the fastest of three, in turn
-        t = {True: [], False: []}
-        for _ in range(3):
-            for on in (True, False):
-                _set_lines(L, plan, on)
-                t[on].append(_time(L, plan, scratch, steps))
-        best = {on: min(v, key=sum) for on, v in t.items()}
-        if verbose:
-            print("autotune line tables: %s ms against %s" % (best[True], best[False]), flush=True)
-        cfg["lines"] = sum(best[True]) < sum(best[False])
-        if cfg["lines"]:
-            cfg["ms"] = best[True]
-        _set_lines(L, plan, cfg["lines"])
     _memo[key] = cfg
     if use_cache:
         _store_cache(key, cfg)
+    cfg = _with_lines(L, plan, cfg, scratch, steps, verbose) if lines else dict(cfg)
     torch.cuda.synchronize()
     return cfg
+
+
+def _with_lines(L, plan, cfg, scratch, steps, verbose):
+    """cfg with whether the plan's line tables are faster than its shapes, which is
+    set on the plan: each side the fastest of three, in turn."""
+    t = {True: [], False: []}
+    for _ in range(3):
+        for on in (True, False):
+            _set_lines(L, plan, on)
+            t[on].append(_time(L, plan, scratch, steps))
+    best = {on: min(v, key=sum) for on, v in t.items()}
+    if verbose:
+        print("autotune line tables: %s ms against %s" % (best[True], best[False]), flush=True)
+    on = sum(best[True]) < sum(best[False])
+    _set_lines(L, plan, on)
+    return dict(cfg, lines=on, ms=best[on])
 
 
 def _apply(L, plan, cfg, strict=True):
