@@ -34,8 +34,8 @@ SEGS = (2, 4, 8, 16, 32)
 LINES = (8, 16, 32, 64)
 MAX_BLOCK = 512
 # Per-voxel coefficients (plan modes 2 and 3) have fixed shapes up to these
-# axis lengths: nothing to choose there.
-DENSE_X, DENSE_YZ = 256, 512
+# axis lengths (y, z: in fields below 4 GiB): nothing to choose there.
+DENSE_X, DENSE_YZ, DENSE_YZ_CELLS = 256, 512, 1 << 29
 
 _memo = {}
 
@@ -129,10 +129,13 @@ def tune(ADI_params, T=None, steps=4, use_cache=True, verbose=False):
            "z": (info["z_seg"], info["z_lines"])}
     best_ms = [None, None, None]
     dense = info["mode"] in (2, 3)
+    fixed = {"x": dense and nx <= DENSE_X}
+    for a, n in (("y", ny), ("z", nz)):
+        fixed[a] = dense and n <= DENSE_YZ and nz * ny * nx < DENSE_YZ_CELLS
     for axis_name, idx, cands in (("x", 0, x_candidates(nx)), ("y", 1, strided_candidates(ny)),
                                   ("z", 2, strided_candidates(nz))):
         results = []
-        if dense and (nx <= DENSE_X if axis_name == "x" else (nz, ny)[idx == 1] <= DENSE_YZ):
+        if fixed[axis_name]:
             cands = [cur[axis_name]]
         for cand in cands:
             trial = dict(cur)

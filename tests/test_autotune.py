@@ -78,3 +78,16 @@ def test_line_tables_are_judged_on_each_plan(library, fresh):
     m = len(library.timed)
     assert m > n and autotune.tune(_params("b", lines=0), T)["lines"] is False
     assert len(library.timed) == m
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+@pytest.mark.parametrize("shape,chosen", [((512, 512, 256), ""), ((512, 512, 257), "x"),
+                                          ((513, 512, 256), "z"), ((40, 520, 300), "xy"),
+                                          ((512, 1024, 1023), "xy"), ((512, 1024, 1024), "xyz")],
+                         ids=lambda s: s if isinstance(s, str) else "x".join(map(str, s)))
+def test_per_voxel_axes_with_shapes_to_choose(library, mode, shape, chosen):
+    """Long axes, and y and z of any length in fields of 4 GiB and more, which the
+    fixed shapes do not serve."""
+    autotune.tune(_params("p", shape, mode, 0), torch.zeros(4, dtype=torch.float64))
+    tried = {a: {tuple(c[a]) for c in library.shapes} for a in "xyz"}
+    assert "".join(a for a in "xyz" if len(tried[a]) > 1) == chosen
