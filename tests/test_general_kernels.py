@@ -1,13 +1,60 @@
 """The general sweep kernels on per-voxel coefficients: what the fixed shapes
-for short axes leave to them."""
+for short axes leave to them (rows of more than 256 cells, columns of more than
+512, fields of 4 GiB)."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
-from heatsim2_amd import _lib
+import oracle
+from heatsim2_amd import _lib, autotune
+from hs2_cases import oracle_coef
+from test_dense import _plan, _problem
+from test_gpu_parity import _curved_case, _every_launch_shape
 
 pytestmark = pytest.mark.gpu
+
+SHAPES = [(5, 6, 257), (4, 5, 300), (8, 4, 512), (3, 4, 513), (2, 3, 1000), (4, 2, 1024),
+          (513, 2, 5), (600, 3, 17), (1024, 2, 9), (2, 520, 6), (2, 1000, 33), (2, 1024, 8)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_every_launch_shape_per_side(shape):
+    """Curved bodies: every launch shape of the long axis against the oracle, with
+    sources and without."""
+    import heatsim2_amd as hs
+    case = _curved_case(shape, seed=5 + sum(shape))
+    case["nsteps"] = 6
+    _every_launch_shape(hs, case)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_every_launch_shape_symmetric(shape):
+    """The same on coefficients with one conductance per face, strongly coupled,
+    with a source field in the first step."""
+    p = _problem(shape, 1)
+    gp = _plan(p)
+    L = _lib.load()
+    rows = oracle_coef(p["M"], p["w"], *p["g"])
+    ref = [oracle.fast_step(rows, p["T0"], p["S"])]
+    ref.append(oracle.fast_step(rows, ref[0], None))
+    info = _lib.plan_info(gp.plan)
+    base = {"x": (info["x_cpl"], info["x_lanes"], info["x_lines"], info["x_lines_y"]),
+            "y": (info["y_seg"], info["y_lines"]), "z": (info["z_seg"], info["z_lines"])}
+    S = torch.from_numpy(p["S"]).cuda()
+    for axis, cands in (("x", autotune.x_candidates(shape[2])),
+                        ("y", autotune.strided_candidates(shape[1])),
+                        ("z", autotune.strided_candidates(shape[0]))):
+        for cand in cands:
+            autotune._apply(L, gp.plan, dict(base, **{axis: cand}))
+            T = torch.from_numpy(p["T0"]).cuda()
+            for n in range(2):
+                _lib.check("hs2_step", L.hs2_step(gp.plan, _lib.ptr(T), _lib.ptr(T), None, None,
+                                                  0, _lib.ptr(S) if n == 0 else None, None,
+                                                  _lib.stream_handle()))
+                assert np.abs(T.cpu().numpy() - ref[n]).max() <= 1e-12 * np.abs(ref[n]).max(), \
+                    (axis, cand, n)
 
 
 @pytest.mark.parametrize("asym", [False, True], ids=["symmetric", "per side"])
