@@ -64,7 +64,7 @@ struct BatchInst {
   double dz;
 };
 
-enum BatchRule { RULE_ALL = 0, RULE_FWD = 1, RULE_RECOMP = 2, RULE_BWD = 3, RULE_SEG = 4 };
+enum BatchRule { RULE_FWD, RULE_RECOMP, RULE_BWD, RULE_SEG };
 
 struct BatchMap {
   const BatchInst *inst;
@@ -95,10 +95,6 @@ __device__ __forceinline__ bool batch_locate(const BatchMap &m, BatchInst &I, in
   const int i = m.blk_inst[gb];
   local = gb - m.blk0[i];
   I = m.inst[i];
-  if (m.rule == RULE_ALL) {
-    t = 0;
-    return true;
-  }
   if (m.rule == RULE_FWD) {
     t = m.ctr[0] + m.j;
     return t < I.nsteps;
@@ -131,7 +127,7 @@ __device__ __forceinline__ DenseView offset_view(DenseView v, long long off) {
 
 namespace hs2 {
 struct AdjGroup;
-// launchers (hs2_kernels.hip, hs2_adjoint.hip); nblocks = this kind's block total
+// launchers (hs2_dense.hip, hs2_adjoint.hip); nblocks = this kind's block total
 // the x sweep; with ck != nullptr (forward) T^t is copied into the instance's
 // checkpoint slot on a checkpoint step; ry as for a plan's sweeps
 hipError_t launch_batch_rows(const BatchMap &m, int nblocks, const DenseView &v, const double *Tn,

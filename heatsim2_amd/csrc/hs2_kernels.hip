@@ -718,11 +718,6 @@ __global__ __launch_bounds__(G *LPB) void k_sweep_x2(Grid g, V view,
 // line stride nx*ny.  Solves (M - La/2) X = M Y - (La/2) T^n along each line.
 // X may alias Y or T^n: a block owns whole lines, and all of its loads
 // happen before its first barrier and all of its stores after its last.
-//
-// FLAT (batched instances): block bx covers CW consecutive columns of all the
-// instance's lines taken in memory order (axis 0: the (j, i) plane, axis 1:
-// the (k, i) columns), and by is P, the segments per line; P x CW may fall
-// short of the block, whose remaining threads only take part in barriers.
 template <class V, int SEG, int AXIS, bool FULL = false, bool RY = false>
 __device__ __forceinline__ void sweep_strided_body(Grid g, V view, int CW, const double *Tn,
                                                    const double *Y, double *X, double *surf,
