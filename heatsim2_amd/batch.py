@@ -9,8 +9,9 @@ counterpart).
 Every instance has its own grid (axes up to 128 cells), step count,
 per-voxel coefficients (per_voxel_coefficients of heatsim2_amd.adjoint) and
 source field applied at its src_step.  The HIP library runs all of them in
-one launch per sweep, with the time loop captured as a HIP graph; the
-results equal what adjoint.surface_history gives for each instance alone.
+groups, one launch per sweep of a group, with the time loop captured as a HIP
+graph; the results equal what adjoint.surface_history gives for each instance
+alone, to round-off.
 """
 import ctypes
 

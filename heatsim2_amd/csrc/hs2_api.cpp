@@ -786,7 +786,11 @@ hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
 
 // Line tables of the plan's axes (hs2_lines.h), where they pay:
 //   kMostBytes   the distinct lines' factors of an axis: they are read by every
-//                block, beside the field, from an XCD's 4 MB of L2;
+//                block, beside the field, from an XCD's 4 MB of L2 (24 kinds of
+//                row at random, the most that fit at 512 cells: 128 x 256 x 256 x
+//                36.2 us against 27.7 with two and 40.9 for the class kernel,
+//                100 x 312 x 512 92 against 77 and 102; 256 kinds of column in
+//                tiles of 16, 40 x 256 x 256: z 12.2 as with four, 18.3);
 //   kMostGroups  groups of 16 like columns over what 16 columns each would
 //                make (128 x 256 x 256, thin spots at random: z 32.1 us at
 //                1.1, 35.1 at 1.25 and 37.1 at 1.5 against 35.5 for the class
@@ -794,10 +798,11 @@ hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
 //   kMostVarying the share of rows whose explicit numbers vary along them,
 //                kMostCells the bytes of those numbers (61 x 149 x 203: x
 //                15.3 us without such rows, 17.7 with half of them alike, 24.4
-//                with 32 MB of them, against 26.3 for the class kernel).  In
-//                rows of more than 512 cells a third is too much already
-//                (100 x 500 x 600: x 284 us at a fifth, 304 at 0.3, 325 at 0.4
-//                against 250; y, which has tables only with x's, gains 50).
+//                with 32 MB of them, against 26.3 for the class kernel; 100 x
+//                300 x 384: 47.7, and 70 with 27 MB, against 82).  In rows of
+//                more than 512 cells a third is too much already (100 x 500 x
+//                600: x 284 us at a fifth, 304 at 0.3, 325 at 0.4 against 250;
+//                y, which reads a field less after x on tables, gains 50).
 // Where the class kernel hands y its right-hand side too (x_ry_ok: whole lines of
 // 16-cell lanes), its source-free x sweep is half as fast again as where it
 // does not, and steps without sources use the tables only (rows_plain) with
@@ -807,7 +812,7 @@ hipError_t distinct_lines(hs2_plan *p, int which, int lines, int len, int most,
 //   - a third of the rows varying at most (128 x 256 x 256: 36.5 at 0.3, 39.2 at
 //     0.4 against 37.4),
 //   - beyond 512 cells, where a line's factors (40 KB) come from L2 for every row,
-//     kPlainRows rows at most (1024 cells: a step 175 us at 16000 rows against 206
+//     kPlainRows rows at most (1024 cells: a step 175 us at 16000 rows against 216
 //     with the class kernel's x, 269 at 20000 against 283, 455 at 31200 against
 //     435), and where any vary kPlainVarying (x 8.6 at 384 against 9.2, 11.2 at
 //     528 against 10.8, 51 at 7808 against 39; 81 at 16000 against 97, which is
@@ -1609,7 +1614,7 @@ int hs2_batch_create(const hs2_batch_inst *in, int ninst, int ckpt_every, hs2_ba
   auto *b = new (std::nothrow) hs2_batch();
   if (!b) return fail(HS2_E_ALLOC, "hs2_batch_create: out of host memory");
   b->ninst = ninst;
-  b->K = (ckpt_every + 1) & ~1;  // even: every segment starts on the same adjoint buffer
+  b->K = (ckpt_every + 1) & ~1;  // even, as the header has it
   long long off = 0, hoff = 0, ck = 0;
   for (int i = 0; i < ninst; i++) {
     const hs2_batch_inst &s = in[i];

@@ -284,11 +284,11 @@ __device__ __forceinline__ double scan_down(double v, const double *b, unsigned 
 // costs three row loads (y-1, y+1 and the next plane) and one store.  No
 // right-hand side is staged and no class byte is read.  Bound by the row
 // loads through L1 and L2 at large sizes (256^3: 56 us, 4.8 TB/s of 16 B per
-// cell, against 72 for the staged class kernel; 128 x 512 x 512: 145 us
+// cell, against 72 for the staged class kernel; 128 x 512 x 512: 137 us
 // against 198), by latency at small ones (61 x 149 x 203: 12.1 against 25
 // us, 40^3: 3.8 against 5.6).  The factors are read from LDS for every row: in
 // registers they cost a wave per SIMD (61 us at 256^3).  Lanes of more than 6
-// cells do worse than two waves per row (512 cells: 178 us against 145): their
+// cells do worse than two waves per row (512 cells: 178 us against 145 then): their
 // loads are 64 bytes apart, and too few waves fit; rows put in lane order
 // through LDS made whole-line loads and stores of it (170 us there, but 60 at
 // 256^3).  Waves in flight weigh most: two rows to a wave (a third of the row
@@ -519,6 +519,7 @@ __global__ __launch_bounds__(256) void k_rows(Grid g, RowTab t, const double *__
 }
 
 // ------------------------------------------------- telling lines apart
+// the finaliser of SplitMix64 (Steele, Lea, Flood 2014)
 __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   x ^= x >> 30;
   x *= 0xbf58476d1ce4e5b9ull;
