@@ -875,13 +875,62 @@ hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int o
   if (!rg) return hipSuccess;
   const int nrow = g.nz * g.ny, nc = 2 * hs2::row_pairs(t.cpl);
   int most = (int)std::min<size_t>(32767, kMostBytes / (sizeof(double) * rg * nc));
-  if ((e = distinct_lines(p, 2, nrow, g.nx, most, &id, &first, &bytes, &count)) != hipSuccess)
+  std::vector<uint8_t> xbytes;
+  int nline = 0;
+  if ((e = distinct_lines(p, 2, nrow, g.nx, most, &id, &first, &xbytes, &nline)) != hipSuccess)
+    return e;
+  if (!nline) return hipSuccess;
+  std::vector<uint32_t> rid(id.begin(), id.end());
+  // the rows' explicit parts: uniform rows keep six numbers, varying ones six
+  // per cell
+  if ((e = distinct_lines(p, 3, nrow, 5 * g.nx, 32767, &id, &first, &bytes, &count)) != hipSuccess)
     return e;
   if (!count) return hipSuccess;
-  std::vector<double> lane((size_t)count * rg * nc), M(g.nx), w(g.nx), gm(g.nx);
+  auto numbers = [&](int c, int i, double *o) {
+    const uint8_t *b = &bytes[(size_t)c * 5 * g.nx];
+    const bool lastj = first[c] % g.ny == g.ny - 1, lastk = first[c] / g.ny == g.nz - 1;
+    const double *ex = entry(2, b[i]);
+    o[0] = ex[0];
+    o[1] = ex[1] * entry(1, b[g.nx + i])[2];
+    o[2] = lastj ? 0.0 : ex[1] * entry(1, b[2 * g.nx + i])[2];
+    o[3] = ex[1] * entry(0, b[3 * g.nx + i])[2];
+    o[4] = lastk ? 0.0 : ex[1] * entry(0, b[4 * g.nx + i])[2];
+    o[5] = ex[1];
+  };
+  // whether the tables serve the plan, before they are built
+  const size_t per = (size_t)rg * t.cpl * hs2::kRowExpl;
+  std::vector<uint32_t> eid(count);
+  uint32_t nplain = 0, nvary = 0;
   for (int c = 0; c < count; c++) {
+    double o[hs2::kRowExpl], f[hs2::kRowExpl];
+    numbers(c, 0, f);
+    bool same = true;
+    for (int i = 1; i < g.nx && same; i++) {
+      numbers(c, i, o);
+      same = std::memcmp(o, f, sizeof f) == 0;
+    }
+    eid[c] = same ? nplain++ : nvary++ | hs2::kRowVaries;
+  }
+  if (sizeof(double) * per * nvary > kMostCells) return hipSuccess;
+  int varying = 0;
+  for (int r = 0; r < nrow; r++) {
+    rid[r] |= eid[id[r]] << 16;
+    varying += (eid[id[r]] & hs2::kRowVaries) != 0;
+  }
+  if (varying > nrow * (g.nx > 512 ? 0.3 : kMostVarying)) return hipSuccess;
+  std::vector<double> row((size_t)nplain * hs2::kRowExpl), cell(per * nvary, 0.0);
+  for (int c = 0; c < count; c++) {
+    const uint32_t q = eid[c] & ~hs2::kRowVaries;
+    if (q == eid[c]) {
+      numbers(c, 0, &row[(size_t)q * hs2::kRowExpl]);
+    } else {
+      for (int i = 0; i < g.nx; i++) numbers(c, i, &cell[per * q + (size_t)i * hs2::kRowExpl]);
+    }
+  }
+  std::vector<double> lane((size_t)nline * rg * nc), M(g.nx), w(g.nx), gm(g.nx);
+  for (int c = 0; c < nline; c++) {
     for (int q = 0; q < g.nx; q++) {
-      const double *v = entry(2, bytes[(size_t)c * g.nx + q]);
+      const double *v = entry(2, xbytes[(size_t)c * g.nx + q]);
       M[q] = v[0];
       w[q] = v[1];
       gm[q] = v[2];
@@ -889,46 +938,6 @@ hipError_t build_lines(hs2_plan *p, const std::vector<double> &tabs, const int o
     hs2::factor_row(g.nx, t.cpl, rg, M.data(), w.data(), gm.data(), &lane[(size_t)c * rg * nc],
                     &t.scan);
   }
-  std::vector<uint32_t> rid(id.begin(), id.end());
-  // the rows' explicit parts: uniform rows keep six numbers, varying ones six
-  // per cell
-  const size_t per = (size_t)rg * t.cpl * hs2::kRowExpl;
-  if ((e = distinct_lines(p, 3, nrow, 5 * g.nx, 32767, &id, &first, &bytes, &count)) != hipSuccess)
-    return e;
-  if (!count) return hipSuccess;
-  std::vector<double> row, cell;
-  std::vector<uint32_t> eid(count);
-  for (int c = 0; c < count; c++) {
-    const uint8_t *b = &bytes[(size_t)c * 5 * g.nx];
-    const bool lastj = first[c] % g.ny == g.ny - 1, lastk = first[c] / g.ny == g.nz - 1;
-    std::vector<double> v(per, 0.0);
-    bool same = true;
-    for (int i = 0; i < g.nx; i++) {
-      const double *ex = entry(2, b[i]);
-      double *o = &v[(size_t)i * hs2::kRowExpl];
-      o[0] = ex[0];
-      o[1] = ex[1] * entry(1, b[g.nx + i])[2];
-      o[2] = lastj ? 0.0 : ex[1] * entry(1, b[2 * g.nx + i])[2];
-      o[3] = ex[1] * entry(0, b[3 * g.nx + i])[2];
-      o[4] = lastk ? 0.0 : ex[1] * entry(0, b[4 * g.nx + i])[2];
-      o[5] = ex[1];
-      if (i > 0) same &= std::memcmp(o, &v[0], sizeof(double) * hs2::kRowExpl) == 0;
-    }
-    if (same) {
-      eid[c] = (uint32_t)(row.size() / hs2::kRowExpl);
-      row.insert(row.end(), v.begin(), v.begin() + hs2::kRowExpl);
-    } else {
-      if (sizeof(double) * (cell.size() + per) > kMostCells) return hipSuccess;
-      eid[c] = (uint32_t)(cell.size() / per) | hs2::kRowVaries;
-      cell.insert(cell.end(), v.begin(), v.end());
-    }
-  }
-  int varying = 0;
-  for (int r = 0; r < nrow; r++) {
-    rid[r] |= eid[id[r]] << 16;
-    varying += (eid[id[r]] & hs2::kRowVaries) != 0;
-  }
-  if (varying > nrow * (g.nx > 512 ? 0.3 : kMostVarying)) return hipSuccess;
   if ((e = keep_lines(p, lane, &t.lane)) != hipSuccess ||
       (e = keep_lines(p, row, &t.row)) != hipSuccess ||
       (e = keep_lines(p, cell, &t.cell)) != hipSuccess ||
